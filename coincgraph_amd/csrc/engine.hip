@@ -3095,7 +3095,7 @@ struct cig_engine {
     // serves the next update group.
     void query_emit(uint32_t k, const QueryOut *outs, size_t nouts, CopyLane &L) {
         const uint32_t stride = (k + 3u) & ~3u;
-        k_ms_gather<<<grid_small, 256, 0, L.stream>>>(ms_dist.p, n, stride, k, ms_out.p);
+        k_ms_gather<0><<<grid_small, kBlock, 0, L.stream>>>(ms_dist.p, n, stride, k, ms_out.p);
         HIPCHK(hipGetLastError());
         uint64_t at = 0;
         for (size_t i = 0; i < nouts; ++i) {
@@ -3147,7 +3147,7 @@ struct cig_engine {
         if (bfs) fill32(reinterpret_cast<uint32_t *>(m.seen), uint64_t(n) * 2, 0);
         fill32(m.stamp, n, 0);
         query_run(algo, sources, k, m);
-        k_ms_gather<<<grid_small, 256, 0, stream>>>(m.dist, n, stride, k, dist_dev);
+        k_ms_gather<0><<<grid_small, kBlock, 0, stream>>>(m.dist, n, stride, k, dist_dev);
         HIPCHK(hipGetLastError());
         end_call(st, 4);
     }
@@ -3296,8 +3296,8 @@ struct cig_engine {
             const uint64_t words = uint64_t(n) * msk;
             if (bytes < words * 4) throw HipError(CIG_EINVAL, "output buffer too small (nsrc * n words)");
             if (ms_out.count < words) ms_out.alloc(words);
-            k_msi_gather<<<grid_small, 256, 0, stream>>>(msi_st.p, n, msk, field == CIG_FIELD_VALUE ? 0u : 1u,
-                                                         ms_out.p);
+            if (field == CIG_FIELD_VALUE) k_ms_gather<1><<<grid_small, kBlock, 0, stream>>>(msi_st.p, n, msk, msk, ms_out.p);
+            else k_ms_gather<2><<<grid_small, kBlock, 0, stream>>>(msi_st.p, n, msk, msk, ms_out.p);
             HIPCHK(hipGetLastError());
             copy_out(out, ms_out.p, words * 4);
             return;

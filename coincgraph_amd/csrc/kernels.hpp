@@ -2415,12 +2415,36 @@ __global__ __launch_bounds__(kBlock) void k_ms_tiles(MsArgs a, uint32_t seq) {
     out_flush(out);
 }
 
-// Source-major result: out[s * n + v] = dist[v][s].
-__global__ void k_ms_gather(const uint32_t *dist, uint32_t n, uint32_t stride, uint32_t k, uint32_t *out) {
-    const uint64_t total = uint64_t(n) * k;
-    for (uint64_t i = gthread(); i < total; i += gthreads()) {
-        const uint32_t s = uint32_t(i / n), v = uint32_t(i % n);
-        out[i] = dist[uint64_t(v) * stride + s];
+// Source-major result: out[s * n + v] = the word of (v, s) in `src`, whose
+// vertex-major rows hold `stride` elements. FIELD: 0 = 32-bit words
+// (distances), 1 / 2 = the value (high) / parent (low) half of 64-bit state
+// words. A workgroup turns tiles of 64 vertices around in LDS, so both sides
+// move whole lines: bound by HBM. Element by element in output order, each
+// 4-B read fetched a line of its own and each element paid two 64-bit
+// divisions (64 sources of 200,003 vertices, 102 MB moved: 224 us, now about 22).
+template <int FIELD>
+__global__ __launch_bounds__(kBlock) void k_ms_gather(const void *src, uint32_t n, uint32_t stride, uint32_t k,
+                                                      uint32_t *out) {
+    __shared__ uint32_t tile[kWave][kWave + 1];  // a column walks all banks
+    const uint32_t lane = lane_id(), w = wave_in_block();
+    uint32_t kw = 1;  // lanes of a vertex when reading
+    while (kw < k) kw <<= 1;
+    const uint32_t s = lane & (kw - 1), sub = lane / kw, vpw = kWave / kw;
+    const uint32_t ntiles = (n + kWave - 1) / kWave;
+    for (uint32_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+        const uint32_t v0 = t * kWave, nv = min(uint32_t(kWave), n - v0);
+#pragma unroll 4
+        for (uint32_t v = w * vpw + sub; v < kWave; v += kWavesPerBlock * vpw) {
+            if (v >= nv || s >= k) continue;
+            const uint64_t at = uint64_t(v0 + v) * stride + s;
+            if constexpr (FIELD == 0) tile[v][s] = static_cast<const uint32_t *>(src)[at];
+            else tile[v][s] = static_cast<const uint32_t *>(src)[2 * at + (FIELD == 1 ? 1 : 0)];
+        }
+        __syncthreads();
+#pragma unroll 4
+        for (uint32_t j = w; j < k; j += kWavesPerBlock)
+            if (lane < nv) out[uint64_t(j) * n + v0 + lane] = tile[lane][j];
+        __syncthreads();
     }
 }
 

@@ -416,15 +416,5 @@ __global__ void k_msi_clear(MsiArgs a) {
     }
 }
 
-// Source-major result: out[s * n + v] = value (field 0) or parent (field 1).
-__global__ void k_msi_gather(const unsigned long long *st, uint32_t n, uint32_t k, uint32_t field, uint32_t *out) {
-    const uint64_t total = uint64_t(n) * k;
-    for (uint64_t i = gthread(); i < total; i += gthreads()) {
-        const uint32_t s = uint32_t(i / n), v = uint32_t(i % n);
-        const unsigned long long x = st[uint64_t(v) * k + s];
-        out[i] = field == 0 ? uint32_t(x >> 32) : uint32_t(x);
-    }
-}
-
 }  // namespace dev
 }  // namespace cig
