@@ -727,6 +727,214 @@ __device__ void expand_tiles(const Op &op, const ExpandCfg &cfg, const Tile *til
     }
 }
 
+// -------------------------------------------------- multi-source expansion
+// Up to 64 sources share the rows of a pass: vertex v is expanded for the
+// sources in a 64-bit mask. The work items of a wave are the (edge, source
+// group) pairs of its rows, a group being GB consecutive sources with at
+// least one bit set, edge-major: consecutive lanes take the groups of one
+// edge, whose per-source words lie next to each other at the destination, so
+// a wave reads whole lines and no lane idles whatever the masks and row
+// lengths are. (A lane per edge that walks the sources instead reads one
+// word of 64 different lines per load.) The slots themselves are read ahead
+// into LDS, kPairSlots at a time with all loads in flight together: a
+// host-tier slot costs a trip over the host link (serving under a 30% budget:
+// 15.3 ms a pass, 16.0 with each item loading its own slot). 128 slots keep
+// six workgroups' LDS on a CU: 16-source SSSP over 2^20 vertices 9.2 ms, 9.5
+// with 512.
+constexpr uint32_t kPairSlots = 128;
+template <int NG>
+struct PairLds {
+    uint32_t pref[kWave];   // exclusive scan of the rows' item counts
+    uint32_t spref[kWave];  // and of their slot counts
+    uint32_t v[kWave];
+    uint32_t cnt[kWave];    // groups of the row's mask
+    uint32_t magic[kWave];  // ceil(2^32 / cnt): item / cnt is exact below 2^26 items a row
+    uint32_t offlo[kWave], offhi[kWave];
+    unsigned long long mask[kWave];
+    uint8_t perm[NG > 1 ? kWave : 1][NG];  // the mask's groups in order
+    uint32_t slot[kPairSlots];
+};
+
+// Expands each lane's row part (`len` slots of v's row at `off`, sources
+// `mask`; len 0: none). The operator:
+//   load(v, w, g, x)         the loads edge (v, w) needs for group g, issued
+//                            for U items per lane before any is used
+//   apply(v, w, g, bits, x)  the group's active `bits`; the sources gained at
+//                            w, as mask bits
+//   mark(w, gained)          all the gains of one edge in this step; true to
+//                            append w
+template <int GB, int U, class Op, class Out>
+__device__ void pair_chunk(const Op &op, const Pools &pools, uint32_t v, uint64_t off, uint32_t len,
+                           unsigned long long mask, PairLds<64 / GB> &L, const Out &out) {
+    constexpr int NG = 64 / GB;
+    const uint32_t lane = lane_id();
+    uint32_t c = 0;
+    if (len != 0 && mask != 0ull) {
+        if constexpr (NG == 1) {
+            c = 1;
+        } else {
+            unsigned long long x = mask;
+            if constexpr (GB == 4) {
+                x |= x >> 1;
+                x |= x >> 2;
+                x &= 0x1111111111111111ull;
+            }
+            for (; x; x &= x - 1) L.perm[lane][c++] = uint8_t(uint32_t(__ffsll(x) - 1) / GB);
+        }
+    }
+    const uint32_t items = len * c;
+    const uint32_t incl = wave_incl_scan(items);
+    const uint32_t total = __shfl(incl, kWave - 1, kWave);
+    if (total == 0) return;
+    const uint32_t slots = c ? len : 0u;
+    const uint32_t sincl = NG == 1 ? incl : wave_incl_scan(slots);
+    const uint32_t stotal = __shfl(sincl, kWave - 1, kWave);
+    L.pref[lane] = incl - items;
+    L.spref[lane] = sincl - slots;
+    L.v[lane] = v;
+    L.offlo[lane] = uint32_t(off);
+    L.offhi[lane] = uint32_t(off >> 32);
+    L.mask[lane] = mask;
+    if constexpr (NG > 1) {
+        L.cnt[lane] = c;
+        L.magic[lane] = c > 1 ? 0xFFFFFFFFu / c + 1u : 0u;
+    }
+    wave_lds_sync();
+    for (uint32_t s0 = 0; s0 < stotal; s0 += kPairSlots) {
+        const uint32_t s1 = min(stotal, s0 + kPairSlots);
+#pragma unroll
+        for (uint32_t j = 0; j < kPairSlots / kWave; ++j) {
+            const uint32_t ss = min(s0 + j * kWave + lane, stotal - 1);
+            const uint32_t o = owner_of(L.spref, ss);
+            L.slot[j * kWave + lane] =
+                pools.row((uint64_t(L.offhi[o]) << 32) | L.offlo[o])[ss - L.spref[o]];
+        }
+        wave_lds_sync();
+        // the items of slots [s0, s1)
+        uint32_t i0 = s0, i1 = s1;
+        if constexpr (NG > 1) {
+            uint32_t o = owner_of(L.spref, s0);
+            i0 = L.pref[o] + (s0 - L.spref[o]) * L.cnt[o];
+            i1 = total;
+            if (s1 < stotal) {
+                o = owner_of(L.spref, s1);
+                i1 = L.pref[o] + (s1 - L.spref[o]) * L.cnt[o];
+            }
+        }
+        for (uint32_t k0 = i0; k0 < i1; k0 += kWave * U) {
+            uint32_t src[U], dst[U], grp[U], first[U], last[U];
+            unsigned long long bits[U];
+            typename Op::Loaded x[U];
+#pragma unroll
+            for (int i = 0; i < U; ++i) {
+                const uint32_t k = k0 + uint32_t(i) * kWave + lane;
+                const uint32_t kk = k < i1 ? k : i1 - 1;
+                const uint32_t o = owner_of(L.pref, kk);
+                const uint32_t r = kk - L.pref[o];
+                uint32_t e = r, g = 0;
+                first[i] = last[i] = lane;
+                if constexpr (NG > 1) {
+                    const uint32_t n = L.cnt[o];
+                    e = n == 1 ? r : __umulhi(r, L.magic[o]);
+                    const uint32_t j = r - e * n;
+                    g = L.perm[o][j];
+                    first[i] = lane > j ? lane - j : 0u;  // this edge's lanes in this step
+                    last[i] = min(lane + (n - 1u - j), uint32_t(kWave - 1));
+                }
+                src[i] = L.v[o];
+                grp[i] = g;
+                bits[i] = L.mask[o];
+                if constexpr (NG > 1) bits[i] = (bits[i] >> (g * GB)) & ((1ull << GB) - 1ull);
+                if (k >= i1) bits[i] = 0;
+                dst[i] = L.slot[L.spref[o] + e - s0];
+            }
+#pragma unroll
+            for (int i = 0; i < U; ++i) op.load(src[i], dst[i], grp[i], x[i]);
+            bool push[U];
+#pragma unroll
+            for (int i = 0; i < U; ++i) {
+                unsigned long long gained = bits[i] ? op.apply(src[i], dst[i], grp[i], bits[i], x[i]) : 0ull;
+                push[i] = false;
+                if (__ballot(gained != 0ull) == 0) continue;
+                // the gains of one edge meet in its first lane
+                if constexpr (NG > 1) {
+#pragma unroll
+                    for (uint32_t d = 1; d < uint32_t(NG); d <<= 1) {
+                        const unsigned long long y = __shfl_down(gained, d, kWave);
+                        if (lane + d <= last[i]) gained |= y;
+                    }
+                }
+                push[i] = lane == first[i] && gained != 0ull && op.mark(dst[i], gained);
+            }
+            out_push<U>(out, push, dst);
+        }
+        wave_lds_sync();  // the slots (and at the end the rows) are replaced next
+    }
+}
+
+// The listed vertices whose rows are shorter than cfg.split; longer rows are
+// in the pass's tiles.
+template <int GB, int U, class Op, class Out>
+__device__ void pair_range(const Op &op, const ExpandCfg &cfg, const Row *rows, const uint32_t *items, uint32_t count,
+                           PairLds<64 / GB> &L, const Out &out) {
+    const uint32_t wpb = blockDim.x / kWave;
+    const uint32_t gwave = blockIdx.x * wpb + wave_in_block(), nwaves = gridDim.x * wpb;
+    uint32_t per = kWave;
+    while (per > 1 && uint64_t(per / 2) * nwaves >= count) per >>= 1;
+    for (uint64_t base = uint64_t(gwave) * per; base < count; base += uint64_t(nwaves) * per) {
+        const uint64_t i = base + lane_id();
+        uint32_t v = 0, len = 0;
+        uint64_t off = 0;
+        unsigned long long mask = 0;
+        if (i < min(uint64_t(count), base + per)) {
+            v = items[i];
+            const Row row = rows[v];
+            mask = op.mask(v);
+            len = row.deg < cfg.split ? row.deg : 0u;
+            off = row.off;
+        }
+        pair_chunk<GB, U>(op, cfg.pools, v, off, len, mask, L, out);
+    }
+}
+
+template <int GB, int U, class Op, class Out>
+__device__ void pair_tiles(const Op &op, const ExpandCfg &cfg, const Tile *tiles, uint32_t ntiles,
+                           PairLds<64 / GB> &L, const Out &out) {
+    const uint32_t wpb = blockDim.x / kWave;
+    const uint32_t gwave = blockIdx.x * wpb + wave_in_block(), nwaves = gridDim.x * wpb;
+    for (uint32_t t = gwave; t < ntiles; t += nwaves) {
+        const Tile tile = tiles[t];
+        const bool lead = lane_id() == 0;
+        pair_chunk<GB, U>(op, cfg.pools, tile.v, tile.start, lead ? tile.len : 0u, lead ? op.mask(tile.v) : 0ull, L,
+                          out);
+    }
+}
+
+// Slots per tile of a long row in a multi-source pass, whose slots carry up
+// to 64 sources each: shorter than the single-source tiles, as long as the
+// tile lists' bound (slots / split tiles for rows of at least split slots)
+// allows.
+__host__ __device__ __forceinline__ uint32_t pair_tile_len(const ExpandCfg &c) {
+    return (min(c.tile_len, 2u * c.split) + 3u) & ~3u;
+}
+
+// Cuts this thread's row (when it is long) into tiles; a workgroup-uniform
+// call, one reservation per workgroup.
+__device__ __forceinline__ void pair_cut(const ExpandCfg &cfg, uint32_t v, const Row &row, bool on, Tile *tiles,
+                                         uint32_t *count, uint32_t *scratch) {
+    const uint32_t tl = pair_tile_len(cfg);
+    const uint32_t nt = on && row.deg >= cfg.split ? (row.deg + tl - 1) / tl : 0u;
+    const uint32_t at = block_reserve<uint32_t>(nt, count, scratch);
+    for (uint32_t j = 0; j < nt; ++j) {
+        Tile t;
+        t.start = row.off + uint64_t(j) * tl;
+        t.v = v;
+        t.len = min(tl, row.deg - j * tl);
+        t.payload = t.pad = 0;
+        tiles[at + j] = t;
+    }
+}
+
 // Adds this wave's counters to its statistics shard (one atomic per wave and
 // non-zero counter).
 __device__ __forceinline__ void flush_counters(Counters &ctr, StatShard *stats, uint32_t stage) {

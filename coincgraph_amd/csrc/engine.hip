@@ -283,7 +283,7 @@ struct cig_engine {
     DBuf<uint8_t> gconf, gskip;
     const uint8_t *cur_skip = nullptr;  // cancel flags of the group being applied
     // multi-source queries
-    DBuf<uint32_t> ms_dist, ms_stamp, ms_out;
+    DBuf<uint32_t> ms_dist, ms_out;
     uint8_t *scratch_dev = nullptr;  // this device's copy of the no-allocation scratch array
     // incremental multi-source state (cig_init with 2..64 BFS/SSSP sources)
     uint32_t msk = 0;  // sources kept; 0: the single-source state word
@@ -291,7 +291,7 @@ struct cig_engine {
     DBuf<unsigned long long> msi_st, msi_act, msi_snap, msi_aff, msi_pinv;
     // CC by union-find (CIG_CFG_CC_UNION_REPAIR)
     DBuf<uint32_t> uf, uroot;
-    DBuf<unsigned long long> ms_act, ms_snap, ms_seen;
+    DBuf<unsigned long long> ms_mark, ms_snap;  // act (BFS: reach, two words a vertex); snap
     CopyLane lane;  // large device-to-host results on the engine stream
     DBuf<uint2> hcnts;
     DBuf<DelTile> dtiles;
@@ -2964,25 +2964,15 @@ struct cig_engine {
     // Up to 64 BFS / SSSP sources on the live graph, independent of the
     // engine's own incremental state (which the query leaves unchanged).
     // out[s * n + v] = distance of v from sources[s] (kInf: unreachable).
-    template <int W, int QPL>
+    template <int W>
     void ms_run(MsArgs &a) {
         advance_round(run_chain(
             [&](uint64_t tag, uint32_t seq) {
                 // whole-graph frontiers: the one-shot grid, not the round grid
-                k_ms_consume<<<grid_small, 256, 0, stream>>>(a, prog_dev, tag, seq);
-                k_ms_expand<W, QPL><<<grid_small, kBlock, 0, stream>>>(a, seq);
-                k_ms_tiles<W, QPL><<<grid_small, kBlock, 0, stream>>>(a, seq);
+                k_ms_consume<W == 2><<<grid_small, kBlock, 0, stream>>>(a, prog_dev, tag, seq);
+                k_ms_expand<W><<<grid_small, kBlock, 0, stream>>>(a, seq);
             },
             round_bound(), "multi-source query"));
-    }
-
-    template <int QPL>
-    void ms_dispatch(uint32_t wkind, MsArgs &a) {
-        switch (wkind) {
-        case 0: ms_run<0, QPL>(a); break;
-        case 1: ms_run<1, QPL>(a); break;
-        default: ms_run<2, QPL>(a); break;
-        }
     }
 
     // One caller buffer of a (possibly merged) query: the distances of its
@@ -2999,13 +2989,20 @@ struct cig_engine {
         query(algo, sources, k, &one, 1, st);
     }
 
-    // Working memory of one multi-source run (vertex-major distances, source
-    // masks, BFS reach masks, enqueue stamps).
+    // Working memory of one multi-source run: vertex-major distances, source
+    // masks (act: one word a vertex; BFS: reach, two words) and snapshots.
     struct QueryMem {
         uint32_t *dist;
-        unsigned long long *act, *snap, *seen;
-        uint32_t *stamp;
+        unsigned long long *mark, *snap;
     };
+
+    // What a run reads before it writes it: the distances start at kInf, the
+    // marks at 0 (a snapshot is written by the round that reads it).
+    void query_clear(uint32_t algo, uint32_t k, const QueryMem &mem) {
+        const uint32_t stride = (k + 3u) & ~3u;
+        fill32(mem.dist, uint64_t(n) * stride, kInf);
+        fill32(reinterpret_cast<uint32_t *>(mem.mark), uint64_t(n) * (algo == CIG_ALGO_BFS ? 4 : 2), 0);
+    }
 
     void query_check(uint32_t algo, const uint32_t *sources, uint32_t k) const {
         if (!loaded) throw HipError(CIG_ESTATE, "no graph loaded");
@@ -3017,22 +3014,18 @@ struct cig_engine {
     }
 
     // Seeds the sources and runs the rounds to the fixed point; the caller
-    // has begun the call and set mem's distances to kInf and its masks to 0
-    // (stamps may hold any tag below the current round, or 0).
+    // has begun the call and cleared mem (query_clear).
     void query_run(uint32_t algo, const uint32_t *sources, uint32_t k, const QueryMem &mem) {
         const bool bfs = algo == CIG_ALGO_BFS;
         MsArgs a{};
         a.ctl = ctl.p;
         a.rows = rows.p;
         a.dist = mem.dist;
-        a.act = mem.act;
+        (bfs ? a.reach : a.act) = mem.mark;
         a.snap = mem.snap;
-        a.seen = bfs ? mem.seen : nullptr;
-        a.stamp = mem.stamp;
         a.q0 = q0.p;
         a.q1 = q1.p;
-        a.t0 = t0.p;
-        a.t1 = t1.p;
+        a.tiles = t0.p;
         a.cfg = ecfg(kStagePropagate);
         a.n = n;
         a.stride = (k + 3u) & ~3u;
@@ -3042,12 +3035,9 @@ struct cig_engine {
         k_ms_seed<<<1, 64, 0, stream>>>(a, list, k);
         HIPCHK(hipGetLastError());
         for (int m : {1, 2, 3, 5}) mark(m);
-        const uint32_t wkind = bfs ? 2u : (cfg.weight_mode == CIG_WEIGHT_HASH64 ? 1u : 0u);
-        switch (qpl) {
-        case 1: ms_dispatch<1>(wkind, a); break;
-        case 4: ms_dispatch<4>(wkind, a); break;
-        default: ms_dispatch<2>(wkind, a); break;
-        }
+        if (bfs) ms_run<2>(a);
+        else if (cfg.weight_mode == CIG_WEIGHT_HASH64) ms_run<1>(a);
+        else ms_run<0>(a);
         mark(4);
     }
 
@@ -3071,21 +3061,15 @@ struct cig_engine {
         query_check(algo, sources, k);
         const uint32_t stride = (k + 3u) & ~3u;
         if (ms_dist.count < uint64_t(n) * stride) ms_dist.alloc(uint64_t(n) * stride);
-        if (ms_act.count < n) {
-            ms_act.alloc(n);
+        if (ms_mark.count < 2ull * n) {
+            ms_mark.alloc(2ull * n);
             ms_snap.alloc(n);
-            ms_stamp.alloc(n);
-            fill32(ms_stamp.p, n, 0);
         }
-        const bool bfs = algo == CIG_ALGO_BFS;
-        if (bfs && ms_seen.count < n) ms_seen.alloc(n);
         if (ms_out.count < uint64_t(n) * k) ms_out.alloc(uint64_t(n) * k);
         begin_call(st);
-        fill32(ms_dist.p, uint64_t(n) * stride, kInf);
-        fill32(reinterpret_cast<uint32_t *>(ms_act.p), uint64_t(n) * 2, 0);
-        fill32(reinterpret_cast<uint32_t *>(ms_snap.p), uint64_t(n) * 2, 0);
-        if (bfs) fill32(reinterpret_cast<uint32_t *>(ms_seen.p), uint64_t(n) * 2, 0);
-        query_run(algo, sources, k, QueryMem{ms_dist.p, ms_act.p, ms_snap.p, ms_seen.p, ms_stamp.p});
+        const QueryMem m{ms_dist.p, ms_mark.p, ms_snap.p};
+        query_clear(algo, k, m);
+        query_run(algo, sources, k, m);
         end_call(st, 4);
     }
 
@@ -3106,16 +3090,16 @@ struct cig_engine {
     }
 
     // Byte offsets of a run's working memory inside the no-allocation scratch
-    // array: distances, act, snap, (BFS) seen, stamps, each 256-B aligned.
-    static uint64_t noalloc_layout(uint32_t nv, uint32_t k, bool bfs, uint64_t off[5]) {
+    // array, each 256-B aligned: distances, marks (two words a vertex),
+    // snapshots. The documented size (36 bytes a vertex beside the distances
+    // for BFS, 28 for SSSP) is what a run may need, and is kept as the limit.
+    static uint64_t noalloc_layout(uint32_t nv, uint32_t k, bool bfs, uint64_t off[3]) {
         auto up = [](uint64_t x) { return (x + 255) & ~uint64_t(255); };
-        const uint64_t stride = (k + 3u) & ~3u;
+        const uint64_t stride = (k + 3u) & ~3u, word = up(uint64_t(nv) * 8);
         off[0] = 0;
-        off[1] = up(off[0] + uint64_t(nv) * stride * 4);
-        off[2] = up(off[1] + uint64_t(nv) * 8);
-        off[3] = up(off[2] + uint64_t(nv) * 8);
-        off[4] = up(off[3] + (bfs ? uint64_t(nv) * 8 : 0));
-        return up(off[4] + uint64_t(nv) * 4);
+        off[1] = up(uint64_t(nv) * stride * 4);
+        off[2] = off[1] + (bfs ? 2 : 1) * word;
+        return up(off[1] + (bfs ? 3 : 2) * word + uint64_t(nv) * 4);
     }
 
     // cig_query with every buffer of the run in the device's scratch array
@@ -3126,26 +3110,19 @@ struct cig_engine {
         query_check(algo, sources, k);
         if (!dist_dev || bytes < uint64_t(n) * k * 4) throw HipError(CIG_EINVAL, "output buffer too small");
         const bool bfs = algo == CIG_ALGO_BFS;
-        uint64_t off[5];
+        uint64_t off[3];
         const uint64_t need = noalloc_layout(n, k, bfs, off);
         if (need > CIG_NOALLOC_SCRATCH_BYTES)
             throw HipError(CIG_ELIMIT, "query needs " + std::to_string(need) + " bytes of scratch; the array holds " +
                                            std::to_string(uint64_t(CIG_NOALLOC_SCRATCH_BYTES)));
         if (!scratch_dev) throw HipError(CIG_EINTERNAL, "scratch array address not resolved");
         const uint32_t stride = (k + 3u) & ~3u;
-        QueryMem m{reinterpret_cast<uint32_t *>(scratch_dev + off[0]),
-                   reinterpret_cast<unsigned long long *>(scratch_dev + off[1]),
-                   reinterpret_cast<unsigned long long *>(scratch_dev + off[2]),
-                   bfs ? reinterpret_cast<unsigned long long *>(scratch_dev + off[3]) : nullptr,
-                   reinterpret_cast<uint32_t *>(scratch_dev + off[4])};
+        const QueryMem m{reinterpret_cast<uint32_t *>(scratch_dev + off[0]),
+                         reinterpret_cast<unsigned long long *>(scratch_dev + off[1]),
+                         reinterpret_cast<unsigned long long *>(scratch_dev + off[2])};
         begin_call(st);
-        // the array keeps the last call's contents (of any engine on this GPU):
-        // everything the run reads before writing is cleared, stamps included
-        fill32(m.dist, uint64_t(n) * stride, kInf);
-        fill32(reinterpret_cast<uint32_t *>(m.act), uint64_t(n) * 2, 0);
-        fill32(reinterpret_cast<uint32_t *>(m.snap), uint64_t(n) * 2, 0);
-        if (bfs) fill32(reinterpret_cast<uint32_t *>(m.seen), uint64_t(n) * 2, 0);
-        fill32(m.stamp, n, 0);
+        // the array keeps the last call's contents (of any engine on this GPU)
+        query_clear(algo, k, m);
         query_run(algo, sources, k, m);
         k_ms_gather<0><<<grid_small, kBlock, 0, stream>>>(m.dist, n, stride, k, dist_dev);
         HIPCHK(hipGetLastError());
@@ -3664,10 +3641,9 @@ struct cig_server {
             } else {
                 try {
                     const uint32_t k = [&] { uint32_t t = 0; for (auto &r : batch) t += uint32_t(r->sources.size()); return t; }();
-                    // distances, the source-major copy, act/snap/seen masks and stamps
-                    const uint64_t need = uint64_t(e->n) * (((k + 3) & ~3u) + k) * 4 + uint64_t(e->n) * 28;
-                    const uint64_t held = e->ms_dist.bytes() + e->ms_out.bytes() + e->ms_act.bytes() +
-                                          e->ms_snap.bytes() + e->ms_seen.bytes() + e->ms_stamp.bytes();
+                    // distances, the source-major copy, marks and snapshots
+                    const uint64_t need = uint64_t(e->n) * (((k + 3) & ~3u) + k) * 4 + uint64_t(e->n) * 24;
+                    const uint64_t held = e->ms_dist.bytes() + e->ms_out.bytes() + e->ms_mark.bytes() + e->ms_snap.bytes();
                     if (need + cfg.hbm_reserve > free_hbm() + held) {
                         for (auto &r : batch) fail(r, CIG_ENOMEM);
                         continue;

@@ -2202,142 +2202,102 @@ __global__ void k_pr_amend_delta(PrArgs a, const uint32_t *touched, float sign) 
 // distances per vertex (vertex-major, `stride` words per vertex), act the
 // sources whose distance at the vertex improved since it was last expanded.
 // A round first takes each frontier vertex's mask (k_ms_consume: snap :=
-// act, act := 0), then expands the rows (k_ms_expand): for every edge (u,w)
-// and every source s in snap[u], dist[w][s] = min(dist[w][s],
-// dist[u][s] + w(u,w)); a destination that improved for any source joins
-// the next frontier. Label-correcting per source, so each distance is the
-// exact shortest-path value (unit weights: BFS depth).
+// act, act := 0) and cuts its long rows into tiles, then expands rows and
+// tiles (k_ms_expand): for every edge (u,w) and every source s in snap[u],
+// dist[w][s] = min(dist[w][s], dist[u][s] + w(u,w)); a destination that
+// improved for any source joins the next frontier. A vertex is queued exactly
+// when its act is non-zero, so the lane whose gain finds act zero appends it.
+// Label-correcting per source, so each distance is the exact shortest-path
+// value. Bound by the random 16-B reads of the distances (L2 misses) and by
+// the memory-side atomics; with a lane per edge that walked the sources, and
+// long rows in a third launch, a round of 16 sources over 2^20 vertices took
+// 320 us on average, now about 200 (64-source BFS over 200,003 vertices: 84
+// and 54 us).
 struct MsArgs {
     Ctl *ctl;
     const Row *rows;
     uint32_t *dist;
     unsigned long long *act, *snap;
-    unsigned long long *seen;  // BFS: sources that reached each vertex
-    uint32_t *stamp;
+    unsigned long long *reach;  // BFS, in place of act: (seen, done) per vertex
     uint32_t *q0, *q1;
-    Tile *t0, *t1;
+    Tile *tiles;
     ExpandCfg cfg;
     uint32_t n, stride;
     uint64_t seed;
 };
 
+// A group is four sources: one 16-B load of the row owner's distances and one
+// of the destination's.
 template <int W>
 struct MsOp {
-    const Row *rows;
+    static constexpr int kGroup = 4, kUnroll = 2;
+    struct Loaded {
+        uint4 du, dw;
+    };
     uint32_t *dist;
     unsigned long long *act;
     const unsigned long long *snap;
-    uint32_t *stamp;
-    uint32_t stride, tag;
+    uint32_t stride;
     uint64_t seed;
-    __device__ bool source(uint32_t v, uint32_t, Row &row, uint32_t &pay) const {
-        if (snap[v] == 0ull) return false;
-        row = rows[v];
-        pay = 0;
-        return row.deg != 0;
+    __device__ unsigned long long mask(uint32_t v) const { return snap[v]; }
+    __device__ void load(uint32_t u, uint32_t w, uint32_t g, Loaded &x) const {
+        x.du = *reinterpret_cast<const uint4 *>(dist + uint64_t(u) * stride + 4u * g);
+        x.dw = *reinterpret_cast<const uint4 *>(dist + uint64_t(w) * stride + 4u * g);
     }
-    __device__ bool tile_source(const Tile &t, uint32_t &pay) const {
-        pay = 0;
-        return snap[t.v] != 0ull;
-    }
-    __device__ uint64_t peek(uint32_t) const { return 0; }
-    // Sources are taken eight at a time: their 16 distance loads are in
-    // flight together and the minimums are non-returning atomics. A source
-    // counts as improved when its candidate beat the value read; if another
-    // lane lowered it further meanwhile, w is merely expanded once more for
-    // that source with its (smaller) current distance, which changes nothing.
-    __device__ bool edge(uint32_t u, uint32_t, uint32_t w, uint64_t) const {
+    // A source counts as improved when its candidate beat the value read; if
+    // another lane lowered it further meanwhile, w is merely expanded once
+    // more for that source with its (smaller) current distance.
+    __device__ unsigned long long apply(uint32_t u, uint32_t w, uint32_t g, unsigned long long bits,
+                                        const Loaded &x) const {
         const uint32_t wt = weight<W>(u, w, seed);
-        const uint32_t *du = dist + uint64_t(u) * stride;
-        uint32_t *dw = dist + uint64_t(w) * stride;
-        unsigned long long gained = 0;
-        for (unsigned long long m = snap[u]; m;) {
-            constexpr int kB = 8;
-            uint32_t s[kB], dv[kB], wv[kB];
-            int cnt = 0;
+        uint32_t *dw = dist + uint64_t(w) * stride + 4u * g;
+        const uint32_t du[4] = {x.du.x, x.du.y, x.du.z, x.du.w}, cur[4] = {x.dw.x, x.dw.y, x.dw.z, x.dw.w};
+        uint32_t gained = 0;
 #pragma unroll
-            for (int k = 0; k < kB; ++k) {
-                s[k] = m ? uint32_t(__ffsll(m) - 1) : 0u;
-                cnt += m ? 1 : 0;
-                m &= m - 1;
-            }
-#pragma unroll
-            for (int k = 0; k < kB; ++k) {
-                dv[k] = k < cnt ? du[s[k]] : kInf;
-                wv[k] = k < cnt ? dw[s[k]] : 0u;
-            }
-#pragma unroll
-            for (int k = 0; k < kB; ++k) {
-                const uint64_t c = uint64_t(dv[k]) + wt;
-                if (k < cnt && c < wv[k]) {  // also rejects c >= kInf
-                    __hip_atomic_fetch_min(&dw[s[k]], uint32_t(c), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    gained |= 1ull << s[k];
-                }
+        for (int i = 0; i < 4; ++i) {
+            const uint64_t c = uint64_t(du[i]) + wt;
+            if (((uint32_t(bits) >> i) & 1u) && c < cur[i]) {  // also rejects c >= kInf
+                __hip_atomic_fetch_min(&dw[i], uint32_t(c), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                gained |= 1u << i;
             }
         }
-        if (!gained) return false;
-        atomicOr(&act[w], gained);
-        return claim(stamp, w, tag);
+        return static_cast<unsigned long long>(gained) << (4u * g);
     }
+    __device__ bool mark(uint32_t w, unsigned long long gained) const { return atomicOr(&act[w], gained) == 0ull; }
 };
 
-// BFS from up to 64 sources, bit-parallel: the rounds are level-synchronous
-// (a round expands exactly the bits its vertices gained in the previous
-// round, all at the same depth), so a destination's depth for source s is
-// fixed the first time bit s reaches it. One 64-bit atomicOr on seen[w] per
-// edge finds the newly reached sources; each (w, s) depth is written once by
-// the lane that set the bit. Same depths as the per-source relaxation.
+// BFS from up to 64 sources, bit-parallel (one group): the rounds are
+// level-synchronous (a round expands exactly the bits its vertices gained in
+// the previous round, all at the same depth), so a destination's depth for
+// source s is fixed when bit s first reaches it, and the next round's consume
+// phase, which knows the depth, writes it for all of the vertex's new bits
+// with whole-line stores. reach[2w] holds the sources that reached w,
+// reach[2w+1] those among them that a consume phase has taken: the first
+// atomicOr of a round that adds a bit finds the two equal and appends w.
 struct MsBfsOp {
-    const Row *rows;
-    uint32_t *dist;
-    unsigned long long *act, *seen;
+    static constexpr int kGroup = 64, kUnroll = 4;
+    struct Loaded {
+        ulonglong2 r;  // seen, done (seen only grows: a stale read under-reports it)
+    };
+    unsigned long long *reach;
     const unsigned long long *snap;
-    uint32_t *stamp;
-    uint32_t stride, tag;
-    // payload: the depth of the row owner's expanding sources, plus one
-    __device__ uint32_t depth_after(uint32_t v) const {
-        const uint32_t s = uint32_t(__ffsll(snap[v]) - 1);
-        return dist[uint64_t(v) * stride + s] + 1u;
+    __device__ unsigned long long mask(uint32_t v) const { return snap[v]; }
+    __device__ void load(uint32_t, uint32_t w, uint32_t, Loaded &x) const {
+        x.r = *reinterpret_cast<const ulonglong2 *>(reach + 2ull * w);
     }
-    __device__ bool source(uint32_t v, uint32_t, Row &row, uint32_t &pay) const {
-        if (snap[v] == 0ull) return false;
-        row = rows[v];
-        pay = depth_after(v);
-        return row.deg != 0;
+    __device__ unsigned long long apply(uint32_t, uint32_t w, uint32_t, unsigned long long bits, const Loaded &x) const {
+        if (!(bits & ~x.r.x)) return 0ull;
+        const unsigned long long old = atomicOr(&reach[2ull * w], bits);
+        return old == x.r.y ? bits & ~old : 0ull;
     }
-    __device__ bool tile_source(const Tile &t, uint32_t &pay) const {
-        if (snap[t.v] == 0ull) return false;
-        pay = depth_after(t.v);
-        return true;
-    }
-    // seen bits only grow, so a stale read can only under-report them
-    __device__ uint64_t peek(uint32_t w) const { return seen[w]; }
-    __device__ bool edge(uint32_t u, uint32_t depth, uint32_t w, uint64_t cur) const {
-        const unsigned long long bits = snap[u] & ~(unsigned long long)cur;
-        if (!bits) return false;
-        const unsigned long long gained = bits & ~atomicOr(&seen[w], bits);
-        if (!gained) return false;
-        uint32_t *dw = dist + uint64_t(w) * stride;
-        for (unsigned long long m = gained; m; m &= m - 1) dw[__ffsll(m) - 1] = depth;
-        atomicOr(&act[w], gained);
-        return claim(stamp, w, tag);
-    }
+    __device__ bool mark(uint32_t, unsigned long long) const { return true; }
 };
 
 template <int W>
-struct MsOpOf {
-    using type = MsOp<W>;
-    __device__ static MsOp<W> make(const MsArgs &a, uint32_t tag) {
-        return MsOp<W>{a.rows, a.dist, a.act, a.snap, a.stamp, a.stride, tag, a.seed};
-    }
-};
-template <>
-struct MsOpOf<2> {
-    using type = MsBfsOp;
-    __device__ static MsBfsOp make(const MsArgs &a, uint32_t tag) {
-        return MsBfsOp{a.rows, a.dist, a.act, a.seen, a.snap, a.stamp, a.stride, tag};
-    }
-};
+__device__ __forceinline__ auto ms_op(const MsArgs &a) {
+    if constexpr (W == 2) return MsBfsOp{a.reach, a.snap};
+    else return MsOp<W>{a.dist, a.act, a.snap, a.stride, a.seed};
+}
 
 // The sources of a multi-source run, passed by value (256 B of kernel
 // arguments), so that no device copy of them is needed.
@@ -2349,69 +2309,100 @@ __global__ void k_ms_seed(MsArgs a, SrcList sources, uint32_t k) {
     const uint32_t r = a.ctl->round;
     for (uint32_t s = gthread(); s < k; s += gthreads()) {
         const uint32_t v = sources.v[s];
-        a.dist[uint64_t(v) * a.stride + s] = 0;
-        atomicOr(&a.act[v], 1ull << s);
-        if (a.seen) atomicOr(&a.seen[v], 1ull << s);
-        if (claim(a.stamp, v, r)) {
+        if (!a.reach) a.dist[uint64_t(v) * a.stride + s] = 0;
+        if (atomicOr(a.reach ? &a.reach[2ull * v] : &a.act[v], 1ull << s) == 0ull) {
             const uint32_t at = atomicAdd(&a.ctl->qcount[r % 3], 1u);
             ((r & 1) ? a.q1 : a.q0)[at] = v;
         }
     }
 }
 
-// Round round+seq-1, phase 1: snapshot and clear the masks of the frontier.
-__global__ void k_ms_consume(MsArgs a, uint64_t *prog, uint64_t tag, uint32_t seq) {
+// Writes `depth` to the distances of v's sources in `mask`, for the 64
+// (v, mask) pairs the wave's lanes hold: 16 B per lane, a row's lanes together.
+__device__ __forceinline__ void ms_write_depths(uint32_t *dist, uint32_t stride, uint32_t v, unsigned long long mask,
+                                                uint32_t depth) {
+    if (__ballot(mask != 0ull) == 0) return;
+    const uint32_t lane = lane_id(), quads = stride / 4;
+    uint32_t g = 1;  // lanes per vertex
+    while (g < quads) g <<= 1;
+    const uint32_t q = lane & (g - 1);
+    for (uint32_t i = lane / g; i < uint32_t(kWave); i += kWave / g) {
+        const uint32_t vv = __shfl(v, int(i), kWave);
+        const unsigned long long mm = __shfl(mask, int(i), kWave);
+        const uint32_t nib = q < quads ? uint32_t(mm >> (4u * q)) & 15u : 0u;
+        uint32_t *d = dist + uint64_t(vv) * stride + 4u * q;
+        if (nib == 15u) {
+            *reinterpret_cast<uint4 *>(d) = make_uint4(depth, depth, depth, depth);
+        } else if (nib) {
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+                if ((nib >> j) & 1u) d[j] = depth;
+        }
+    }
+}
+
+// Round round+seq-1, phase 1: snapshot and clear the masks of the frontier,
+// cut its long rows into tiles (so that phase 2 expands rows and tiles of one
+// round in one launch); BFS: write the depths of the bits taken.
+template <bool BFS>
+__global__ __launch_bounds__(kBlock) void k_ms_consume(MsArgs a, uint64_t *prog, uint64_t tag, uint32_t seq) {
+    __shared__ uint32_t scratch[kMaxWavesPerBlock + 1];
     Ctl *c = a.ctl;
     const uint32_t r = c->round + seq - 1;
     const uint32_t nq = c->qcount[r % 3];
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         c->qcount[(r + 2) % 3] = 0;
-        c->scount = 0;
+        c->tcount[(r + 2) % 3] = 0;
         if (nq) c->rounds += 1;
         post_progress(prog, tag, nq != 0);
     }
     const uint32_t *qin = (r & 1) ? a.q1 : a.q0;
-    for (uint32_t i = gthread(); i < nq; i += gthreads()) {
-        const uint32_t v = qin[i];
-        a.snap[v] = atomicExch(&a.act[v], 0ull);
+    Counters ctr;
+    for (uint32_t base = blockIdx.x * blockDim.x; base < nq; base += gthreads()) {
+        const uint32_t i = base + threadIdx.x;
+        const bool on = i < nq;
+        uint32_t v = 0;
+        Row row{};
+        unsigned long long m = 0;
+        if (on) {
+            v = qin[i];
+            row = a.rows[v];
+            if constexpr (BFS) {
+                const ulonglong2 x = *reinterpret_cast<const ulonglong2 *>(a.reach + 2ull * v);
+                m = x.x & ~x.y;
+                a.reach[2ull * v + 1] = x.x;
+            } else {
+                m = a.act[v];
+                a.act[v] = 0ull;
+            }
+            a.snap[v] = m;
+            ctr.scanned += row.deg;
+            ctr.vexp += row.deg ? 1 : 0;
+            if (row.off & kHostTier) ctr.host += row.deg;
+        }
+        pair_cut(a.cfg, v, row, on, a.tiles, &c->tcount[r % 3], scratch);
+        if constexpr (BFS) ms_write_depths(a.dist, a.stride, v, m, seq - 1);
     }
+    if (nq) flush_counters(ctr, a.cfg.stats, a.cfg.stage);
 }
 
-// Phase 2: expand the frontier rows; rows of at least `split` slots become
-// tiles for phase 3 of the same round, so every part of a row is expanded
-// with the same snapshot.
-template <int W, int QPL>
+// Phase 2: expand the frontier's rows and tiles.
+template <int W>
 __global__ __launch_bounds__(kBlock) void k_ms_expand(MsArgs a, uint32_t seq) {
-    __shared__ WaveLds lds[kWavesPerBlock];
-    __shared__ RoundStage stage;
+    using Op = decltype(ms_op<W>(a));
+    __shared__ PairLds<64 / Op::kGroup> lds[kWavesPerBlock];
+    __shared__ PullStage stage;
     Ctl *c = a.ctl;
     const uint32_t r = c->round + seq - 1;
     const uint32_t nq = c->qcount[r % 3];
     if (nq == 0) return;
-    const auto op = MsOpOf<W>::make(a, r + 1);
-    Counters ctr;
-    const uint32_t *qin = (r & 1) ? a.q1 : a.q0;
-    const StagedOut<2048, 128> out{Sink{(r & 1) ? a.q0 : a.q1, &c->qcount[(r + 1) % 3]},
-                                   TileSink{a.t0, &c->scount}, &stage};
+    const Op op = ms_op<W>(a);
+    const StagedOut<1024, 2> out{Sink{(r & 1) ? a.q0 : a.q1, &c->qcount[(r + 1) % 3]}, TileSink{nullptr, &c->scount},
+                                 &stage};
     out_init(out);
-    expand_range<QPL>(op, a.cfg, qin, nq, out, lds[wave_in_block()], ctr);
-    flush_counters(ctr, a.cfg.stats, a.cfg.stage);
-    out_flush(out);
-}
-
-// Phase 3: the tiles cut in phase 2.
-template <int W, int QPL>
-__global__ __launch_bounds__(kBlock) void k_ms_tiles(MsArgs a, uint32_t seq) {
-    __shared__ RoundStage stage;
-    Ctl *c = a.ctl;
-    const uint32_t r = c->round + seq - 1;
-    const uint32_t nt = c->scount;
-    if (nt == 0) return;
-    const auto op = MsOpOf<W>::make(a, r + 1);
-    const StagedOut<2048, 128> out{Sink{(r & 1) ? a.q0 : a.q1, &c->qcount[(r + 1) % 3]},
-                                   TileSink{nullptr, &c->scount}, &stage};
-    out_init(out);
-    expand_tiles<QPL>(op, a.cfg, a.t0, nt, out);
+    PairLds<64 / Op::kGroup> &L = lds[wave_in_block()];
+    pair_range<Op::kGroup, Op::kUnroll>(op, a.cfg, a.rows, (r & 1) ? a.q1 : a.q0, nq, L, out);
+    pair_tiles<Op::kGroup, Op::kUnroll>(op, a.cfg, a.tiles, c->tcount[r % 3], L, out);
     out_flush(out);
 }
 
