@@ -2327,11 +2327,9 @@ struct cig_engine {
         x.snap = msi_snap.p;
         x.affm = msi_aff.p;
         x.pinv = msi_pinv.p;
-        x.stamp = stamp.p;
         x.q0 = q0.p;
         x.q1 = q1.p;
-        x.t0 = t0.p;
-        x.t1 = t1.p;
+        x.tiles = t0.p;
         x.alist = alist.p;
         x.cfg = ecfg(kStagePropagate);
         x.dels = d;
@@ -2369,7 +2367,6 @@ struct cig_engine {
         fill32(reinterpret_cast<uint32_t *>(msi_st.p), uint64_t(n) * k * 2, kInf);
         for (auto *b : {&msi_act, &msi_snap, &msi_aff, &msi_pinv})
             fill32(reinterpret_cast<uint32_t *>(b->p), uint64_t(n) * 2, 0);
-        fill32(stamp.p, n, 0);
         msk = k;
         ms_sources.assign(sources, sources + k);
         SrcList list{};
@@ -2378,80 +2375,72 @@ struct cig_engine {
         HIPCHK(hipGetLastError());
     }
 
-    template <int W, int QPL>
-    void msi_relax_qpl(uint32_t grid) {
+    // Multi-source rounds carry up to 64 sources per row: four workgroups per
+    // CU (as many as their LDS admits), where a single-source round takes one
+    // (64 sources, 2^18 vertices, 4 + 4 batches: 13.7 ms with one, 13.0 with
+    // four, 13.2 with six).
+    uint32_t grid_msi() const { return std::max(grid_round, uint32_t(cus) * 4); }
+
+    template <int W>
+    void msi_relax_w() {
         MsiArgs a = msi_args(nullptr, 0, nullptr, 0);
         advance_round(run_chain(
             [&](uint64_t tag, uint32_t seq) {
-                k_msi_consume<<<grid_small, 256, 0, stream>>>(a, a.act, prog_dev, tag, seq);
-                timed_round([&] { k_msi_expand<W, false, QPL><<<grid, kBlock, 0, stream>>>(a, seq); });
-                k_msi_tiles<W, false, QPL><<<grid, kBlock, 0, stream>>>(a, seq);
+                k_msi_consume<<<grid_msi(), kBlock, 0, stream>>>(a, a.act, prog_dev, tag, seq);
+                timed_round([&] { k_msi_expand<W, false><<<grid_msi(), kBlock, 0, stream>>>(a, seq); });
             },
             round_bound(), "multi-source fixed point"));
         HIPCHK(hipGetLastError());
     }
 
-    template <int W>
-    void msi_relax_w(uint32_t grid) {
-        switch (qpl) {
-        case 1: msi_relax_qpl<W, 1>(grid); break;
-        case 4: msi_relax_qpl<W, 4>(grid); break;
-        default: msi_relax_qpl<W, 2>(grid); break;
-        }
-    }
-
-    void msi_relax(uint32_t grid) {
+    void msi_relax() {
         switch (weight_kind()) {
-        case 0: msi_relax_w<0>(grid); break;
-        case 1: msi_relax_w<1>(grid); break;
-        default: msi_relax_w<2>(grid); break;
+        case 0: msi_relax_w<0>(); break;
+        case 1: msi_relax_w<1>(); break;
+        default: msi_relax_w<2>(); break;
         }
     }
 
     // Invalidation waves to their fixed point, then the reset that also lists
     // every affected vertex.
-    template <int QPL>
     void msi_invalidate(const MsiArgs &x) {
         MsiArgs a = x;
         a.cfg = ecfg(kStageInvalidate);
-        k_msi_inval_seed<<<grid_small, 256, 0, stream>>>(a);
+        k_msi_inval_seed<<<grid_small, kBlock, 0, stream>>>(a);
         HIPCHK(hipGetLastError());
         advance_round(run_chain(
             [&](uint64_t tag, uint32_t seq) {
-                k_msi_consume<<<grid_small, 256, 0, stream>>>(a, a.pinv, prog_dev, tag, seq);
-                k_msi_expand<0, true, QPL><<<grid_round, kBlock, 0, stream>>>(a, seq);
-                k_msi_tiles<0, true, QPL><<<grid_round, kBlock, 0, stream>>>(a, seq);
+                k_msi_consume<<<grid_msi(), kBlock, 0, stream>>>(a, a.pinv, prog_dev, tag, seq);
+                k_msi_expand<0, true><<<grid_msi(), kBlock, 0, stream>>>(a, seq);
             },
             round_bound(), "multi-source invalidation"));
         k_msi_reset<<<grid_small, 256, 0, stream>>>(a);
         HIPCHK(hipGetLastError());
     }
 
-    template <int W, int QPL>
+    template <int W>
     void msi_repair(const MsiArgs &x) {
         MsiArgs a = x;
         a.cfg = ecfg(kStageRepair);
         mark(8);
-        k_msi_repair<W, QPL><<<grid_small, kBlock, 0, stream>>>(a);
+        k_msi_repair<W><<<grid_small, kBlock, 0, stream>>>(a);
         mark(9);
         scan_timed = stages_now;
-        k_msi_repair_tiles<W, QPL><<<grid_small, kBlock, 0, stream>>>(a);
-        k_msi_repair_done<<<grid_small, 256, 0, stream>>>(a);
+        k_msi_repair_tiles<W><<<grid_small, kBlock, 0, stream>>>(a);
+        k_msi_repair_done<<<grid_small, kBlock, 0, stream>>>(a);
         HIPCHK(hipGetLastError());
     }
 
     template <int W>
     void msi_deletes(const MsiArgs &x) {
-        switch (qpl) {
-        case 1: msi_invalidate<1>(x); mark(2); msi_repair<W, 1>(x); break;
-        case 4: msi_invalidate<4>(x); mark(2); msi_repair<W, 4>(x); break;
-        default: msi_invalidate<2>(x); mark(2); msi_repair<W, 2>(x); break;
-        }
+        msi_invalidate(x);
+        mark(2);
+        msi_repair<W>(x);
     }
 
     template <int W>
     void msi_insert_seed(const MsiArgs &x, bool skip_affected) {
-        k_msi_insert_seed<W><<<grid_small, 256, 0, stream>>>(x, skip_affected ? 1u : 0u);
+        k_msi_insert_seed<W><<<grid_small, kBlock, 0, stream>>>(x, skip_affected ? 1u : 0u);
         HIPCHK(hipGetLastError());
     }
 
@@ -2471,7 +2460,7 @@ struct cig_engine {
             mutate_apply(m);
             const MsiArgs xd = msi_args(d, nd, nullptr, 0);
             msi_deletes<W>(xd);
-            msi_relax(grid_round);
+            msi_relax();
             msi_clear();
             mutate_finish(m, false);
             // stage 2: the adds
@@ -2481,13 +2470,13 @@ struct cig_engine {
             mutate_apply(ma);
             const MsiArgs xa = msi_args(nullptr, 0, a, na);
             msi_insert_seed<W>(xa, false);
-            msi_relax(grid_round);
+            msi_relax();
             mark(4);
             end_call(st, 0);
             if (hctl.p->overflow_cnt) {
                 recover_overflow(ma);
                 msi_insert_seed<W>(xa, false);
-                msi_relax(grid_round);
+                msi_relax();
                 end_call(st, 0);
             }
             mutate_finish(ma);
@@ -2506,11 +2495,7 @@ struct cig_engine {
             if (side_claims) mutate_claims(m, side);
             HIPCHK(hipEventRecord(join_ev, side));
             try {
-                switch (qpl) {
-                case 1: msi_invalidate<1>(x); break;
-                case 4: msi_invalidate<4>(x); break;
-                default: msi_invalidate<2>(x); break;
-                }
+                msi_invalidate(x);
             } catch (...) {
                 (void)hipStreamSynchronize(side);
                 throw;
@@ -2519,11 +2504,7 @@ struct cig_engine {
             HIPCHK(hipStreamWaitEvent(stream, join_ev, 0));
             mutate_apply(m, side_claims);
             mark(1);
-            switch (qpl) {
-            case 1: msi_repair<W, 1>(x); break;
-            case 4: msi_repair<W, 4>(x); break;
-            default: msi_repair<W, 2>(x); break;
-            }
+            msi_repair<W>(x);
         } else {
             mutate_group(m);
             mutate_apply(m);
@@ -2534,13 +2515,13 @@ struct cig_engine {
         mark(3);
         if (na) msi_insert_seed<W>(x, nd != 0);
         mark(5);
-        msi_relax(grid_round);
+        msi_relax();
         mark(4);
         end_call(st, 4);
         if (na && hctl.p->overflow_cnt) {
             recover_overflow(m);
             msi_insert_seed<W>(x, false);
-            msi_relax(grid_round);
+            msi_relax();
             end_call(st, 4);
         }
         defer_finish(m, false);
@@ -2633,7 +2614,7 @@ struct cig_engine {
         begin_call(st);
         for (int k : {1, 2, 3, 5}) mark(k);
         if (is_pr()) pr_converge();
-        else if (msk) msi_relax(grid_small);
+        else if (msk) msi_relax();
         else if (uf_mode()) uf_all();
         else relax();
         mark(4);
