@@ -61,6 +61,8 @@ struct Ctl {
     // fixed-point rounds (relax / PR); slot = absolute round % 3
     alignas(kCtlLine) uint32_t qcount[3];
     alignas(kCtlLine) uint32_t tcount[3];
+    uint32_t fscan[3];     // PR: slot's frontier is flags only (a pull pass added to it)
+    alignas(kCtlLine) uint32_t flist[3];   // PR: list entries written by the scan of such a frontier
     uint32_t round;        // next absolute round to run
     uint32_t converged;
     alignas(kCtlLine) uint32_t done;  // workgroups finished in the current round kernel
@@ -86,8 +88,7 @@ struct Ctl {
     alignas(kCtlLine) uint32_t ht_cursor;     // and their table slots
     uint32_t pr_invalid;
     alignas(kCtlLine) uint32_t group_cursor;  // records grouped so far (< 2^32 per call)
-    uint32_t pl_tiles;      // PR pull plan: tiles of long incoming rows
-    uint32_t pl_multi;      // PR pull plan: rows of more than one tile
+    uint32_t plan[9];       // PR pull plan: length of each list (kPlanLists)
     uint32_t pull_rounds;   // PR rounds of the current call run in pull form
     uint32_t amend_pull;    // PR batch amendment gathers (1) or scatters (amend_push = 1)
     uint32_t amend_push;

@@ -205,8 +205,11 @@ constexpr uint32_t kQplDefault = 2;  // quads (4 slots) per lane and step
 // all incoming rows costs less than scattering with atomics from a frontier
 // of n/4096 hub-heavy vertices.)
 constexpr uint32_t kPullDivisorDefault = 4096;
+// The mask pays where the contributions' lines come from HBM: at 2^22
+// vertices (16 MB of contributions) a masked sweep takes 350 us, 270 without.
 constexpr uint32_t kPullMaskDivisor = 4;
-constexpr uint32_t kPullBlocksPerCu = 64;
+constexpr uint32_t kPullMaskMin = 1u << 24;
+constexpr uint32_t kPullBlocksPerCu = 8;
 
 }  // namespace
 
@@ -258,6 +261,8 @@ struct cig_engine {
     // PR pull plan: tiles of long incoming rows, rows of several tiles, partial sums
     DBuf<Tile> ptiles;
     DBuf<PullRow> prow;
+    DBuf<PullEntry> pent;
+    DBuf<uint32_t> pcnt;
     DBuf<float> tpart;
     DBuf<unsigned long long> fl_off;  // host-tier free blocks by class (FreeList), when the tier holds rows
     DBuf<int> fl_cnt;
@@ -1031,9 +1036,11 @@ struct cig_engine {
             a.in_rows = in_rows_p();
             a.ptiles = ptiles.p;
             a.prow = prow.p;
+            a.pent = pent.p;
+            a.pcnt = pcnt.p;
             a.tpart = tpart.p;
             a.amask = amask.p;
-            a.mask_max = std::max<uint32_t>(1u, n / kPullMaskDivisor);
+            a.mask_max = n > kPullMaskMin ? std::max<uint32_t>(1u, n / kPullMaskDivisor) : 0u;
             a.odeg = odeg.p;
         }
         return a;
@@ -1048,6 +1055,8 @@ struct cig_engine {
         // sized by n: a later cig_load_csr may bring a larger graph
         if (amask.count < (uint64_t(n) + 63) / 64) amask.alloc((uint64_t(n) + 63) / 64);
         if (odeg.count < n) odeg.alloc(n);
+        if (pent.count < n) pent.alloc(n);
+        if (!pcnt.p) pcnt.alloc(kPlanBlocks * kPlanLists);
         if (need <= ptile_cap) return;
         ptiles.alloc(need);
         tpart.alloc(need);
@@ -1083,16 +1092,8 @@ struct cig_engine {
             k_pr_degrees<<<grid_small, 256, 0, stream>>>(rows.p, n, odeg.p);
             advance_round(run_chain(
                 [&](uint64_t tag, uint32_t seq) {
-                    k_pr_consume<<<grid_pull, kBlock, 0, stream>>>(a, prog_dev, tag, seq);
-                    k_pr_scatter<1><<<grid_round, kBlock, 0, stream>>>(a, seq);
-                    timed_round([&] {
-                        switch (qpl) {
-                        case 1: k_pr_pull<1><<<grid_pull, kBlock, 0, stream>>>(a, seq); break;
-                        case 4: k_pr_pull<4><<<grid_pull, kBlock, 0, stream>>>(a, seq); break;
-                        default: k_pr_pull<2><<<grid_pull, kBlock, 0, stream>>>(a, seq); break;
-                        }
-                    });
-                    k_pr_pull_long<<<grid_small, kBlock, 0, stream>>>(a, seq);
+                    k_pr_consume<<<grid_small, kBlock, 0, stream>>>(a, prog_dev, tag, seq);
+                    timed_round([&] { pull_sweep(a, seq); });
                 },
                 cfg.pr_max_rounds, "PageRank"));
         }
@@ -2529,15 +2530,14 @@ struct cig_engine {
 
     // ------------------------------------------------------------ PR batch
     void pull_plan(const PrArgs &a, const uint32_t *gate) {
-        k_pr_pull_plan_reset<<<1, 64, 0, stream>>>(ctl.p);
-        k_pr_pull_plan<<<grid_small, kBlock, 0, stream>>>(a, gate);
+        k_pr_plan_count<<<kPlanBlocks, kBlock, 0, stream>>>(a, gate);
+        k_pr_plan_fill<<<kPlanBlocks, kBlock, 0, stream>>>(a, gate);
         HIPCHK(hipGetLastError());
     }
 
-    template <int QPL>
-    void pull_pass(const PrArgs &a, uint32_t seq) {
-        k_pr_pull<QPL><<<grid_pull, kBlock, 0, stream>>>(a, seq);
-        k_pr_pull_long<<<grid_small, kBlock, 0, stream>>>(a, seq);
+    void pull_sweep(const PrArgs &a, uint32_t seq) {
+        if (renum) k_pr_pull<true><<<uint32_t(cus), kPullHubBlock, 0, stream>>>(a, seq);
+        else k_pr_pull<false><<<grid_pull, kBlock, 0, stream>>>(a, seq);
     }
 
     // The touched sources' contribution sign*alpha*x/deg along their current
@@ -2551,11 +2551,8 @@ struct cig_engine {
             fill32(reinterpret_cast<uint32_t *>(amask.p), 2 * ((uint64_t(n) + 63) / 64), 0u);
             k_pr_amend_delta<<<grid_small, 256, 0, stream>>>(a, touched.p, sign);
             pull_plan(a, sign < 0 ? &ctl.p->amend_pull : nullptr);
-            switch (qpl) {
-            case 1: pull_pass<1>(a, 0); break;
-            case 4: pull_pass<4>(a, 0); break;
-            default: pull_pass<2>(a, 0); break;
-            }
+            pull_sweep(a, 0);
+            HIPCHK(hipGetLastError());
         }
         PrScatterOp sc{rows.p, res.p, stamp.p, delta.p, &ctl.p->pr_invalid, cfg.pr_epsilon};
         PrAmendOp op{rows.p, rank.p, sign, n, sc};

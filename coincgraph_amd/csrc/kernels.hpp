@@ -14,6 +14,8 @@ namespace cg = cooperative_groups;
 // LDS staging of the round kernels: 2048 frontier items and 128 tiles per
 // workgroup (19 KB with the wave slots of a 256-thread workgroup).
 using RoundStage = StageLds<2048, 128>;
+// and of kernels that make no tiles: small, so that many workgroups fit on a CU.
+using ListStage = StageLds<1024, 2>;
 
 __device__ __forceinline__ uint64_t next_pow2_dev(uint64_t d) {
     uint64_t c = d < kMinRowCap ? kMinRowCap : d;
@@ -62,7 +64,7 @@ __global__ void k_reset_ctl(Ctl *c, uint32_t flags) {
     for (int i = 0; i < 4; ++i) c->st_edges[i] = c->st_vexp[i] = c->st_host[i] = 0;
     if (!keep_rounds) {
         c->round = 1;
-        for (int i = 0; i < 3; ++i) c->qcount[i] = c->tcount[i] = 0;
+        for (int i = 0; i < 3; ++i) c->qcount[i] = c->tcount[i] = c->fscan[i] = c->flist[i] = 0;
     }
 }
 
@@ -1642,15 +1644,27 @@ __global__ void k_advance_round(Ctl *c, uint32_t by) {
 }
 
 // ---------------------------------------------------------- PageRank rounds
-// Pull plan of one solve: incoming rows at least kPullSplit slots long are cut
-// into tiles of kPullTile slots; a row of several tiles also gets a PullRow
-// whose tiles' partial sums k_pr_pull_long adds up.
-constexpr uint32_t kPullSplit = 256;
+// Pull plan of one solve. Incoming rows of up to kPullSplit slots are listed
+// by size class: class c holds the rows of up to 4 << c slots, which 1 << c
+// lanes read with one 16-B load each. Longer rows are cut into tiles of
+// kPullTile slots; a row of several tiles also gets a PullRow, whose last tile
+// to finish adds the tiles' partial sums up.
+constexpr uint32_t kPullClasses = 7;
+constexpr uint32_t kPullSplit = 4u << (kPullClasses - 1);
 constexpr uint32_t kPullTile = 2048;
 
-struct PullRow {
-    uint32_t v, first, nt, pad;
+struct PullEntry {
+    uint64_t off;
+    uint32_t v, deg;
 };
+
+struct PullRow {
+    uint32_t first, nt, done, pad;
+};
+
+// The plan's lists: the classes, then tiles and rows of several tiles.
+constexpr uint32_t kPlanLists = kPullClasses + 2, kPlanTiles = kPullClasses, kPlanMulti = kPullClasses + 1;
+constexpr uint32_t kPlanBlocks = 512;  // workgroups of the two plan kernels
 
 struct PrArgs {
     Ctl *ctl;
@@ -1666,8 +1680,10 @@ struct PrArgs {
     // least pull_min vertices gather; pull_min = kNone disables it
     const Row *in_rows;
     uint32_t n, pull_min;
+    PullEntry *pent;  // the classes' rows, class by class
     Tile *ptiles;
     PullRow *prow;
+    uint32_t *pcnt;   // plan kernels: per workgroup, the length of each list
     float *tpart;
     // bit v set iff delta[v] != 0; pull passes of rounds with fewer than
     // mask_max frontier vertices (and amendments) test it before gathering
@@ -1772,6 +1788,8 @@ __global__ __launch_bounds__(kBlock) void k_pr_consume(PrArgs a, uint64_t *prog,
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         c->qcount[(r + 2) % 3] = 0;
         c->tcount[(r + 2) % 3] = 0;
+        c->fscan[(r + 2) % 3] = 0;
+        c->flist[(r + 2) % 3] = 0;
         if (nq) c->rounds += 1;
         post_progress(prog, tag, nq != 0);
     }
@@ -1808,15 +1826,26 @@ __global__ __launch_bounds__(kBlock) void k_pr_consume(PrArgs a, uint64_t *prog,
         flush_counters(ctr, a.cfg.stats, a.cfg.stage);
         return;
     }
-    const uint32_t *qin = (r & 1) ? a.q1 : a.q0;
+    uint32_t *qin = (r & 1) ? a.q1 : a.q0;
     Tile *tiles = (r & 1) ? a.t1 : a.t0;
-    for (uint32_t base = blockIdx.x * blockDim.x; base < nq; base += gthreads()) {
-        const uint32_t i = base + threadIdx.x;
+    // a frontier that a pull pass left as flags: this scan writes the list
+    const bool scan = c->fscan[r % 3] != 0;
+    const uint32_t bound = scan ? a.n : nq;
+    for (uint32_t base = blockIdx.x * blockDim.x; base < bound; base += gthreads()) {
+        uint32_t i = base + threadIdx.x;
         uint32_t v = 0, nt = 0;
         Row row{};
         float d = 0.0f;
-        if (i < nq) {
+        bool on = i < bound;
+        if (scan) {
+            v = i;
+            on = on && a.queued[v] != 0u;
+            i = block_reserve<uint32_t>(on ? 1u : 0u, &c->flist[r % 3], scratch);
+            if (on) qin[i] = v;
+        } else if (on) {
             v = qin[i];
+        }
+        if (on) {
             const float rv = a.res[v];
             a.queued[v] = 0u;
             if (!isfinite(rv) || !isfinite(a.rank[v])) atomicExch(&c->pr_invalid, 1u);
@@ -1850,7 +1879,7 @@ __global__ __launch_bounds__(kBlock) void k_pr_consume(PrArgs a, uint64_t *prog,
             if (row.off & kHostTier) ctr.host += row.deg;
             d = 0.0f;
         }
-        if (i < nq) a.delta[i] = d;
+        if (on) a.delta[i] = d;
     }
     flush_counters(ctr, a.cfg.stats, a.cfg.stage);
 }
@@ -1858,13 +1887,11 @@ __global__ __launch_bounds__(kBlock) void k_pr_consume(PrArgs a, uint64_t *prog,
 // PageRank round, scatter phase (pr_residual.cuh:74-100) of round
 // round + seq - 1; the consume phase of the same round posted its progress.
 template <int QPL>
-__global__ __launch_bounds__(kBlock) void k_pr_scatter(PrArgs a, uint32_t seq) {
-    __shared__ WaveLds lds[kWavesPerBlock];
-    __shared__ RoundStage stage;
+__device__ void pr_scatter_round(const PrArgs &a, uint32_t seq, WaveLds &lds, RoundStage &stage) {
     Ctl *c = a.ctl;
     const uint32_t r = c->round + seq - 1;
     const uint32_t nq = c->qcount[r % 3];
-    if (nq == 0 || pr_dense(a, nq)) return;
+    if (nq == 0) return;
     const uint32_t nt = c->tcount[r % 3];
     const uint32_t *qin = (r & 1) ? a.q1 : a.q0;
     Tile *tiles = (r & 1) ? a.t1 : a.t0;
@@ -1874,10 +1901,17 @@ __global__ __launch_bounds__(kBlock) void k_pr_scatter(PrArgs a, uint32_t seq) {
                                    TileSink{tiles, &c->scount}, &stage};
     out_init(out);
     Counters ctr;
-    expand_range<QPL>(op, a.cfg, qin, nq, out, lds[wave_in_block()], ctr);
+    expand_range<QPL>(op, a.cfg, qin, nq, out, lds, ctr);
     expand_tiles<QPL>(op, a.cfg, tiles, nt, out);
     flush_counters(ctr, a.cfg.stats, a.cfg.stage);
     out_flush(out);
+}
+
+template <int QPL>
+__global__ __launch_bounds__(kBlock) void k_pr_scatter(PrArgs a, uint32_t seq) {
+    __shared__ WaveLds lds[kWavesPerBlock];
+    __shared__ RoundStage stage;
+    pr_scatter_round<QPL>(a, seq, lds[wave_in_block()], stage);
 }
 
 // ------------------------------------------------ PageRank rounds, pull form
@@ -1891,23 +1925,93 @@ __global__ __launch_bounds__(kBlock) void k_pr_scatter(PrArgs a, uint32_t seq) {
 // its residual crosses epsilon, as in the scatter. Only the summation order
 // differs from the scatter's (whose atomic order is itself unspecified).
 
-// Builds the pull plan of the current incoming rows (they do not change
-// during a solve); `gate` (when given) must be non-zero for it to run.
-__global__ void k_pr_pull_plan(PrArgs a, const uint32_t *gate) {
-    __shared__ uint32_t scratch[2 * (kMaxWavesPerBlock + 1)];
-    Ctl *c = a.ctl;
+// The pull plan of the current incoming rows (they do not change during a
+// solve), in two launches over the same vertex ranges: k_pr_plan_count counts
+// what each workgroup adds to each list, k_pr_plan_fill adds the counts of the
+// workgroups before it up and writes the lists, so neither needs an atomic on
+// a shared cursor (one per 256 rows and list held the pass to 200 us at 2^22
+// vertices; now 23 and 105). `gate` (when given) must be non-zero to run.
+__device__ __forceinline__ uint32_t plan_range(uint32_t n, uint32_t &end) {
+    const uint32_t per = (uint32_t((uint64_t(n) + kPlanBlocks - 1) / kPlanBlocks) + 255u) & ~255u;
+    const uint64_t lo = uint64_t(blockIdx.x) * per;
+    end = uint32_t(min(uint64_t(n), lo + per));
+    return uint32_t(min(uint64_t(n), lo));
+}
+
+// The list of a row of deg >= 1 slots; tiles: how many it is cut into.
+__device__ __forceinline__ uint32_t plan_list(uint32_t deg, uint32_t &tiles) {
+    tiles = 0;
+    if (deg > kPullSplit) {
+        tiles = (deg + kPullTile - 1) / kPullTile;
+        return kPlanTiles;
+    }
+    return deg <= 4 ? 0u : 30u - uint32_t(__clz(deg - 1));
+}
+
+__device__ __forceinline__ void plan_tally(const Row &row, uint32_t *cnt) {
+    if (row.deg == 0) return;
+    uint32_t tiles;
+    const uint32_t l = plan_list(row.deg, tiles);
+    atomicAdd(&cnt[l], l == kPlanTiles ? tiles : 1u);
+    if (tiles > 1) atomicAdd(&cnt[kPlanMulti], 1u);
+}
+
+__global__ __launch_bounds__(kBlock) void k_pr_plan_count(PrArgs a, const uint32_t *gate) {
+    __shared__ uint32_t cnt[kPlanLists];
     if (gate && *gate == 0) return;
-    for (uint32_t base = blockIdx.x * blockDim.x; base < a.n; base += gthreads()) {
-        const uint32_t v = base + threadIdx.x;
-        Row row{};
-        if (v < a.n) row = a.in_rows[v];
-        const uint32_t nt = row.deg >= kPullSplit ? (row.deg + kPullTile - 1) / kPullTile : 0u;
-        const uint32_t x[2] = {nt, nt > 1 ? 1u : 0u};
-        uint32_t *const cnt[2] = {&c->pl_tiles, &c->pl_multi};
-        uint32_t at[2];
-        block_reserve_n<2>(x, cnt, at, scratch);
-        const uint32_t mi = nt > 1 ? at[1] : kNone;
-        if (nt > 1) a.prow[mi] = PullRow{v, at[0], nt, 0u};
+    if (threadIdx.x < kPlanLists) cnt[threadIdx.x] = 0u;
+    __syncthreads();
+    uint32_t end;
+    for (uint32_t v = plan_range(a.n, end) + threadIdx.x; v < end; v += kBlock) plan_tally(a.in_rows[v], cnt);
+    __syncthreads();
+    if (threadIdx.x < kPlanLists) a.pcnt[blockIdx.x * kPlanLists + threadIdx.x] = cnt[threadIdx.x];
+}
+
+__global__ __launch_bounds__(kBlock) void k_pr_plan_fill(PrArgs a, const uint32_t *gate) {
+    __shared__ uint32_t cur[kPlanLists], tot[kPlanLists];
+    if (gate && *gate == 0) return;
+    const uint32_t lane = lane_id();
+    for (uint32_t l = wave_in_block(); l < kPlanLists; l += kWavesPerBlock) {
+        uint64_t all = 0, before = 0;
+        for (uint32_t w = lane; w < kPlanBlocks; w += kWave) {
+            const uint32_t x = a.pcnt[w * kPlanLists + l];
+            all += x;
+            before += w < blockIdx.x ? x : 0u;
+        }
+        all = wave_sum64(all);
+        before = wave_sum64(before);
+        if (lane == 0) {
+            cur[l] = uint32_t(before);
+            tot[l] = uint32_t(all);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t run = 0;
+        for (uint32_t l = 0; l < kPullClasses; ++l) {  // the classes share one array
+            cur[l] += run;
+            run += tot[l];
+        }
+        if (blockIdx.x == 0)
+            for (uint32_t l = 0; l < kPlanLists; ++l) a.ctl->plan[l] = tot[l];
+    }
+    __syncthreads();
+    uint32_t end;
+    for (uint32_t v = plan_range(a.n, end) + threadIdx.x; v < end; v += kBlock) {
+        const Row row = a.in_rows[v];
+        if (row.deg == 0) continue;
+        uint32_t nt;
+        const uint32_t l = plan_list(row.deg, nt);
+        if (l != kPlanTiles) {
+            a.pent[atomicAdd(&cur[l], 1u)] = PullEntry{row.off, v, row.deg};
+            continue;
+        }
+        const uint32_t at = atomicAdd(&cur[kPlanTiles], nt);
+        uint32_t mi = kNone;
+        if (nt > 1) {
+            mi = atomicAdd(&cur[kPlanMulti], 1u);
+            a.prow[mi] = PullRow{at, nt, 0u, 0u};
+        }
         for (uint32_t j = 0; j < nt; ++j) {
             Tile t;
             t.start = row.off + uint64_t(j) * kPullTile;
@@ -1915,13 +2019,9 @@ __global__ void k_pr_pull_plan(PrArgs a, const uint32_t *gate) {
             t.len = min(kPullTile, row.deg - j * kPullTile);
             t.payload = mi;
             t.pad = 0;
-            a.ptiles[at[0] + j] = t;
+            a.ptiles[at + j] = t;
         }
     }
-}
-
-__global__ void k_pr_pull_plan_reset(Ctl *c) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) c->pl_tiles = c->pl_multi = 0;
 }
 
 __device__ __forceinline__ float wave_sum_f(float x) {
@@ -1930,11 +2030,78 @@ __device__ __forceinline__ float wave_sum_f(float x) {
     return x;
 }
 
-// Adds `sum` to r(w) (w's only writer this round) and reports whether w
-// joins the next frontier.
-__device__ __forceinline__ bool pull_apply(const PrArgs &a, uint32_t w, float sum) {
+// Where a pull pass finds the contributions: the first kPullHubs of them (the
+// hubs of a renumbered engine) in LDS, the others in memory, behind the
+// mask's bit when there is one (the mask is 1/32 of delta's size, so a sparse
+// pass touches far fewer cache lines).
+constexpr uint32_t kPullHubs = 32768;
+constexpr uint32_t kPullHubBlock = 1024;
+constexpr uint32_t kPullSets = 2;
+// an LDS address as such: through a generic pointer the two reads of a slot
+// merge into one flat load, which waits for both memories
+using LdsFloat = __attribute__((address_space(3))) const float;
+template <bool HUB>
+struct PullSrc {
+    const float *delta;
+    const unsigned long long *mask;
+    LdsFloat *hub;
+};
+
+// Sum of delta[] over the live slots of QPL quads whose loads are in flight
+// together; dead slots (past the row's end or past the last quad) add 0. A
+// slot that needs no memory read (a hub, a cleared mask bit) reads word 0, a
+// line its wave shares, so the vector memory unit walks the others only.
+template <int QPL, bool HUB>
+__device__ __forceinline__ void pull_gather(const PullSrc<HUB> &p, const uint32_t (&d)[QPL][4],
+                                            const uint32_t (&live)[QPL], float (&s)[QPL]) {
+    float x[QPL][4];
+    bool need[QPL][4];
+#pragma unroll
+    for (int q = 0; q < QPL; ++q)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) need[q][k] = !HUB || d[q][k] >= kPullHubs;
+    if (p.mask) {
+        uint32_t w[QPL][4];
+        const uint32_t *m32 = reinterpret_cast<const uint32_t *>(p.mask);
+#pragma unroll
+        for (int q = 0; q < QPL; ++q)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) w[q][k] = m32[need[q][k] ? d[q][k] >> 5 : 0u];
+#pragma unroll
+        for (int q = 0; q < QPL; ++q)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const bool on = (w[q][k] >> (d[q][k] & 31u)) & 1u;
+                const float g = p.delta[need[q][k] && on ? d[q][k] : 0u];
+                x[q][k] = on ? g : 0.0f;
+            }
+    } else {
+#pragma unroll
+        for (int q = 0; q < QPL; ++q)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) x[q][k] = p.delta[need[q][k] ? d[q][k] : 0u];
+    }
+    if constexpr (HUB) {
+#pragma unroll
+        for (int q = 0; q < QPL; ++q)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float h = p.hub[need[q][k] ? 0u : d[q][k]];
+                x[q][k] = need[q][k] ? x[q][k] : h;
+            }
+    }
+#pragma unroll
+    for (int q = 0; q < QPL; ++q) {
+        s[q] = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) s[q] += uint32_t(k) < live[q] ? x[q][k] : 0.0f;
+    }
+}
+
+// Adds `sum` to r(w), whose value before the pass is `old` (this lane is w's
+// only writer), and reports whether w joins the next frontier.
+__device__ __forceinline__ bool pull_add(const PrArgs &a, uint32_t w, float old, float sum) {
     if (sum == 0.0f) return false;
-    const float old = a.res[w];
     const float now = old + sum;
     a.res[w] = now;
     if (!isfinite(now)) atomicExch(&a.ctl->pr_invalid, 1u);
@@ -1945,148 +2112,146 @@ __device__ __forceinline__ bool pull_apply(const PrArgs &a, uint32_t w, float su
     return false;
 }
 
-struct PullLds {
-    uint32_t pref[kWave];
-    uint32_t deg[kWave];
-    uint32_t offlo[kWave];
-    uint32_t offhi[kWave];
-    float acc[kWave];
+// A unit of the class lists: kPullSets sets of 64 >> c rows of class c, 1 << c
+// lanes a row, one quad a lane. No search for a slot's row and no shared
+// accumulator: a row's lanes add up by shuffles.
+struct PullAt {
+    uint32_t c, first, end;  // class, first row, end of the class's list (wave-uniform)
+    bool on;
+};
+struct PullRows {
+    PullEntry e[kPullSets];
+    bool on[kPullSets];  // false: past the list's end (e repeats its last row)
+};
+struct PullQuads {
+    uint32_t d[kPullSets][4], live[kPullSets];
+    float old[kPullSets];
 };
 
-// Sum of delta[] over the live slots of QPL quads whose loads are in flight
-// together; dead slots (past the row's end or past the last quad) add 0.
-// With a mask, only sources whose mask bit is set are gathered (the mask is
-// 1/32 of delta's size, so a sparse pass touches far fewer cache lines).
-template <int QPL>
-__device__ __forceinline__ void pull_gather(const float *delta, const unsigned long long *mask,
-                                            const uint32_t (&d)[QPL][4], const uint32_t (&live)[QPL],
-                                            float (&s)[QPL]) {
-    float x[QPL][4];
-    if (mask) {
-        unsigned long long w[QPL][4];
+// Unit u of the lists whose lengths are cnt[].
+__device__ __forceinline__ PullAt pull_at(const uint32_t (&cnt)[kPullClasses], uint32_t u) {
+    PullAt p{0u, 0u, 0u, false};
+    uint32_t base = 0;
 #pragma unroll
-        for (int q = 0; q < QPL; ++q)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) w[q][k] = mask[d[q][k] >> 6];
-#pragma unroll
-        for (int q = 0; q < QPL; ++q)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) x[q][k] = (w[q][k] >> (d[q][k] & 63u)) & 1ull ? delta[d[q][k]] : 0.0f;
-    } else {
-#pragma unroll
-        for (int q = 0; q < QPL; ++q)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) x[q][k] = delta[d[q][k]];
+    for (uint32_t c = 0; c < kPullClasses; ++c) {
+        const uint32_t rows = kPullSets * (kWave >> c), units = (cnt[c] + rows - 1) / rows;
+        if (!p.on && u < units) p = PullAt{c, base + u * rows, base + cnt[c], true};
+        u -= p.on ? 0u : units;
+        base += cnt[c];
     }
+    return p;
+}
+
+__device__ __forceinline__ void pull_load_rows(const PrArgs &a, const PullAt &p, PullRows &r) {
 #pragma unroll
-    for (int q = 0; q < QPL; ++q) {
-        s[q] = 0.0f;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) s[q] += uint32_t(k) < live[q] ? x[q][k] : 0.0f;
+    for (uint32_t s = 0; s < kPullSets; ++s) {
+        const uint32_t i = p.first + s * (kWave >> p.c) + (lane_id() >> p.c);
+        r.on[s] = p.on && i < p.end;
+        r.e[s] = PullEntry{0ull, 0u, 0u};
+        if (p.on) r.e[s] = a.pent[min(i, p.end - 1)];
     }
 }
 
-// The 64 vertices [v0, v0+64): rows shorter than kPullSplit are summed here,
-// lanes walking the wave's concatenated rows quad by quad and adding each
-// quad's sum to its row's LDS accumulator.
-template <int QPL, class Out>
-__device__ void pull_chunk(const PrArgs &a, const unsigned long long *mask, uint32_t v0, PullLds &L,
-                           const Out &out, Counters &ctr) {
-    const uint32_t lane = lane_id();
-    const uint32_t v = v0 + lane;
-    uint32_t deg = 0;
-    uint64_t off = 0;
-    if (v < a.n) {
-        const Row row = a.in_rows[v];
-        if (row.deg < kPullSplit) {
-            deg = row.deg;
-            off = row.off;
+__device__ __forceinline__ void pull_load_quads(const PrArgs &a, const PullAt &p, const PullRows &r, PullQuads &q) {
+    const uint32_t j = lane_id() & ((1u << p.c) - 1u);
+#pragma unroll
+    for (uint32_t s = 0; s < kPullSets; ++s) {
+        const uint32_t deg = r.e[s].deg;
+        const bool in = 4u * j < deg;
+        q.live[s] = 0;
+        q.old[s] = 0.0f;
+        if (p.on) {
+            // wave-uniform; lanes past the row's end read its first quad, whose
+            // slots past deg (never written, any word) are aliased to its first
+            const uint32_t live = load_quad_stream(a.cfg.pools.row(r.e[s].off), in ? j : 0u, deg, q.d[s]);
+            q.live[s] = r.on[s] && in ? live : 0u;
+            q.old[s] = a.res[r.e[s].v];
+        }
+    }
+}
+
+template <bool HUB>
+__device__ __forceinline__ void pull_finish(const PrArgs &a, const PullSrc<HUB> &src, const PullAt &p, const PullRows &r,
+                                            const PullQuads &q, uint32_t &joined, Counters &ctr) {
+    float sum[kPullSets];
+    pull_gather<kPullSets>(src, q.d, q.live, sum);
+    const uint32_t j = lane_id() & ((1u << p.c) - 1u);
+    for (uint32_t dd = (1u << p.c) >> 1; dd > 0; dd >>= 1)
+#pragma unroll
+        for (uint32_t s = 0; s < kPullSets; ++s) sum[s] += __shfl_xor(sum[s], int(dd), kWave);
+#pragma unroll
+    for (uint32_t s = 0; s < kPullSets; ++s) {
+        const PullEntry &e = r.e[s];
+        if (j == 0 && r.on[s]) {
+            ctr.scanned += e.deg;
             ctr.vexp += 1;
+            if (e.off & kHostTier) ctr.host += e.deg;
+            joined += pull_add(a, e.v, q.old[s], sum[s]) ? 1u : 0u;
         }
     }
-    ctr.scanned += deg;
-    if (off & kHostTier) ctr.host += deg;
-    const uint32_t nq = (deg + 3u) >> 2;
-    const uint32_t incl = wave_incl_scan(nq);
-    const uint32_t total = __shfl(incl, kWave - 1, kWave);
-    float sum = 0.0f;
-    if (total) {
-        L.pref[lane] = incl - nq;
-        L.deg[lane] = deg;
-        L.offlo[lane] = uint32_t(off);
-        L.offhi[lane] = uint32_t(off >> 32);
-        L.acc[lane] = 0.0f;
-        wave_lds_sync();
-        for (uint32_t k0 = 0; k0 < total; k0 += kWave * QPL) {
-            uint32_t d[QPL][4], own[QPL], live[QPL];
-#pragma unroll
-            for (int q = 0; q < QPL; ++q) {
-                const uint32_t k = k0 + uint32_t(q) * kWave + lane;
-                const uint32_t kk = k < total ? k : total - 1;
-                own[q] = owner_of(L.pref, kk);
-                const uint64_t o = (uint64_t(L.offhi[own[q]]) << 32) | L.offlo[own[q]];
-                live[q] = load_quad_stream(a.cfg.pools.row(o), kk - L.pref[own[q]], L.deg[own[q]], d[q]);
-                if (k >= total) live[q] = 0;
-            }
-            float s[QPL];
-            pull_gather<QPL>(a.delta, mask, d, live, s);
-#pragma unroll
-            for (int q = 0; q < QPL; ++q)
-                if (live[q]) atomicAdd(&L.acc[own[q]], s[q]);
-        }
-        wave_lds_sync();
-        sum = L.acc[lane];
-        wave_lds_sync();  // LDS is reused by the next chunk of this wave
-    }
-    const bool f[1] = {deg != 0 && pull_apply(a, v, sum)};
-    const uint32_t val[1] = {v};
-    out_push<1>(out, f, val);
 }
 
-// One tile of a long incoming row: a wave sum; a one-tile row is finished
-// here, the tiles of a longer row leave partial sums for k_pr_pull_long.
-template <int QPL, class Out>
-__device__ void pull_tile(const PrArgs &a, const unsigned long long *mask, uint32_t ti, const Out &out,
+// One tile of a long incoming row: all its loads in flight, then the gathers;
+// a wave sum. A one-tile row is finished here; a longer row's tiles leave their
+// partial sums at the memory side (atomics, whose answers order them) and the
+// last one adds them up.
+template <bool HUB>
+__device__ void pull_tile(const PrArgs &a, const PullSrc<HUB> &src, const Tile &t, uint32_t ti, uint32_t &joined,
                           Counters &ctr) {
-    const Tile t = a.ptiles[ti];
+    constexpr int Q = kPullTile / (4 * kWave), P = 2;
     const uint32_t *p = a.cfg.pools.row(t.start);
     const uint32_t lane = lane_id();
     const uint32_t nq = (t.len + 3u) >> 2;
-    float acc = 0.0f;
-    for (uint32_t k0 = 0; k0 < nq; k0 += kWave * QPL) {
-        uint32_t d[QPL][4], live[QPL];
+    uint32_t d[Q][4], live[Q];
 #pragma unroll
-        for (int q = 0; q < QPL; ++q) {
-            const uint32_t k = k0 + uint32_t(q) * kWave + lane;
+    for (int q = 0; q < Q; ++q) {
+        const uint32_t k = uint32_t(q) * kWave + lane;
+        live[q] = 0;
+        if (uint32_t(q) * kWave < nq) {  // wave-uniform
             live[q] = load_quad_stream(p, k < nq ? k : nq - 1, t.len, d[q]);
             if (k >= nq) live[q] = 0;
         }
-        float s[QPL];
-        pull_gather<QPL>(a.delta, mask, d, live, s);
+    }
+    float acc = 0.0f;
 #pragma unroll
-        for (int q = 0; q < QPL; ++q) acc += s[q];
+    for (int q = 0; q < Q; q += P) {
+        if (uint32_t(q) * kWave >= nq) break;
+        uint32_t dd[P][4], ll[P];
+        float s[P];
+#pragma unroll
+        for (int i = 0; i < P; ++i) {
+            ll[i] = live[q + i];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) dd[i][k] = uint32_t(q + i) * kWave < nq ? d[q + i][k] : 0u;
+        }
+        pull_gather<P>(src, dd, ll, s);
+#pragma unroll
+        for (int i = 0; i < P; ++i) acc += s[i];
     }
     acc = wave_sum_f(acc);
     if (lane == 0) {
         ctr.scanned += t.len;
         if (t.start & kHostTier) ctr.host += t.len;
     }
-    bool f[1] = {false};
-    if (t.payload == kNone) {
+    if (t.payload != kNone) {
+        PullRow &pr = a.prow[t.payload];
+        uint32_t last = 0;
         if (lane == 0) {
-            ctr.vexp += 1;
-            f[0] = pull_apply(a, t.v, acc);
+            atomicExch(&a.tpart[ti], acc);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the partial sum has arrived
+            last = atomicAdd(&pr.done, 1u) + 1u == pr.nt ? 1u : 0u;
         }
-    } else if (lane == 0) {
-        a.tpart[ti] = acc;
+        if (!__shfl(last, 0, kWave)) return;
+        acc = 0.0f;
+        for (uint32_t j = lane; j < pr.nt; j += kWave) acc += ld_acquire(&a.tpart[pr.first + j]);
+        acc = wave_sum_f(acc);
+        if (lane == 0) atomicExch(&pr.done, 0u);  // for the next pass
     }
-    const uint32_t val[1] = {t.v};
-    out_push<1>(out, f, val);
+    if (lane == 0) {
+        ctr.vexp += 1;
+        joined += pull_add(a, t.v, a.res[t.v], acc) ? 1u : 0u;
+    }
 }
-
-// Frontier staging of the pull kernels (they make no tiles): small, so that
-// many workgroups fit on a CU and keep many gathers in flight.
-using PullStage = StageLds<1024, 2>;
 
 // Where a pull pass appends and whether it runs. seq >= 1: the scatter phase
 // of round round + seq - 1 when that round is dense, appending to the next
@@ -2096,7 +2261,7 @@ using PullStage = StageLds<1024, 2>;
 struct PullPass {
     bool run;
     uint32_t stage;
-    Sink sink;
+    uint32_t slot;  // of the frontier the vertices join
     const unsigned long long *mask;
 };
 
@@ -2104,66 +2269,113 @@ __device__ __forceinline__ PullPass pull_pass(const PrArgs &a, uint32_t seq) {
     Ctl *c = a.ctl;
     if (seq == 0) {
         const uint32_t r = c->round;
-        return PullPass{c->amend_pull != 0, kStageAmend, Sink{(r & 1) ? a.q1 : a.q0, &c->qcount[r % 3]}, a.amask};
+        return PullPass{c->amend_pull != 0, kStageAmend, r % 3, a.amask};
     }
     const uint32_t r = c->round + seq - 1;
     const uint32_t nq = c->qcount[r % 3];
-    return PullPass{pr_dense(a, nq), kStageRepair, Sink{(r & 1) ? a.q0 : a.q1, &c->qcount[(r + 1) % 3]},
-                    nq < a.mask_max ? a.amask : nullptr};
+    return PullPass{pr_dense(a, nq), kStageRepair, (r + 1) % 3, nq < a.mask_max ? a.amask : nullptr};
 }
 
-// Pull pass `seq` (see pull_pass): short rows by wave chunks, then the plan's tiles.
-template <int QPL>
-__global__ __launch_bounds__(kBlock) void k_pr_pull(PrArgs a, uint32_t seq) {
-    __shared__ PullLds lds[kWavesPerBlock];
-    __shared__ PullStage stage;
-    Ctl *c = a.ctl;
-    const PullPass pass = pull_pass(a, seq);
-    if (!pass.run) return;
-    const StagedOut<1024, 2> out{pass.sink, TileSink{nullptr, &c->scount}, &stage};
-    out_init(out);
-    Counters ctr;
-    const uint32_t wpb = blockDim.x / kWave;
-    const uint32_t gwave = blockIdx.x * wpb + wave_in_block(), nwaves = gridDim.x * wpb;
-    const uint32_t nchunks = (a.n + kWave - 1) / kWave;
-    for (uint32_t ch = gwave; ch < nchunks; ch += nwaves)
-        pull_chunk<QPL>(a, pass.mask, ch * kWave, lds[wave_in_block()], out, ctr);
-    const uint32_t nt = c->pl_tiles;
-    for (uint32_t t = gwave; t < nt; t += nwaves) pull_tile<QPL>(a, pass.mask, t, out, ctr);
-    flush_counters(ctr, a.cfg.stats, pass.stage);
-    out_flush(out);
-}
-
-// Rows of several tiles: a wave adds up the tiles' partial sums.
-__global__ __launch_bounds__(kBlock) void k_pr_pull_long(PrArgs a, uint32_t seq) {
-    __shared__ PullStage stage;
-    Ctl *c = a.ctl;
-    const uint32_t nm = c->pl_multi;
-    const PullPass pass = pull_pass(a, seq);
-    if (nm == 0 || !pass.run) return;
-    const StagedOut<1024, 2> out{pass.sink, TileSink{nullptr, &c->scount}, &stage};
-    out_init(out);
-    const uint32_t wpb = blockDim.x / kWave;
-    const uint32_t gwave = blockIdx.x * wpb + wave_in_block(), nwaves = gridDim.x * wpb;
-    const uint32_t lane = lane_id();
-    uint64_t rows_done = 0;
-    for (uint32_t i = gwave; i < nm; i += nwaves) {
-        const PullRow pr = a.prow[i];
-        float s = 0.0f;
-        for (uint32_t j = lane; j < pr.nt; j += kWave) s += a.tpart[pr.first + j];
-        s = wave_sum_f(s);
-        bool f[1] = {false};
-        if (lane == 0) {
-            rows_done += 1;
-            f[0] = pull_apply(a, pr.v, s);
-        }
-        const uint32_t val[1] = {pr.v};
-        out_push<1>(out, f, val);
+// The vertices that joined the frontier in a pull pass have their queued flag
+// set; the frontier's count takes one atomic per workgroup, and its list is
+// not written (flist = 0): a dense consume scans the flags anyway, a sparse
+// one that finds no list scans them too. (A list cost up to an atomic per
+// chunk on one address.) Every thread of the workgroup must call it.
+__device__ __forceinline__ void pull_count(Ctl *c, const PullPass &pass, uint32_t joined, uint32_t *cnt) {
+    if (threadIdx.x == 0) *cnt = 0u;
+    __syncthreads();
+    const uint32_t s = uint32_t(wave_sum64(joined));
+    if (s && lane_id() == 0) atomicAdd(cnt, s);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (*cnt) atomicAdd(&c->qcount[pass.slot], *cnt);
+        if (blockIdx.x == 0) c->fscan[pass.slot] = 1u;
     }
+}
+
+// What a round does with its contributions, or the amendment's sweep (seq 0;
+// see pull_pass): gather along the incoming rows when the pass is dense, else
+// scatter along the frontier's rows (a sparse round). One launch holds both
+// forms: which one a round takes is known on the device only, and a launch
+// that finds nothing to do costs the round 5 us and a gap.
+//
+// HUB (engines that number vertices by out-degree): one 1024-thread workgroup
+// per CU holds the first 32768 contributions in LDS (R-MAT scale 20: the
+// sources of 70% of the edges, scale 22: of 53%), since a gather from memory
+// moves a 128-B line into L1 for 4 bytes. What bounds it: the lines of the
+// other gathers (scale 22: 31 M, 3.9 GB into L1 per sweep) and the stream of
+// source ids. Per dense sweep, scale 20 / 22: 110 / 285 us with 64 workgroups
+// per CU that wrote the frontier's list, searched every slot's row and added
+// quads up in LDS; now 56 / 265. Two sets of rows in flight per wave: one 62 /
+// 280, four 76 / 335 (their lines displace each other in L1). Without HUB: 81
+// / 360.
+template <bool HUB>
+__global__ __launch_bounds__(HUB ? kPullHubBlock : kBlock) void k_pr_pull(PrArgs a, uint32_t seq) {
+    constexpr uint32_t B = HUB ? kPullHubBlock : kBlock;
+    struct ScatterLds {
+        WaveLds w[B / kWave];
+        RoundStage stage;
+    };
+    union Lds {
+        float hub[HUB ? kPullHubs : 1];
+        ScatterLds scatter;
+        __device__ Lds() {}
+    };
+    __shared__ Lds lds;
+    __shared__ uint32_t total;
+    Ctl *c = a.ctl;
+    const PullPass pass = pull_pass(a, seq);
+    if (!pass.run) {
+        if (seq) pr_scatter_round<1>(a, seq, lds.scatter.w[wave_in_block()], lds.scatter.stage);
+        return;
+    }
+    // Neighbouring units go to different workgroups (the heavy ones are
+    // neighbours). A wave's units are pipelined: a unit's row entries are read
+    // two units ahead, its quads one ahead; the first loads go out before the
+    // hubs are staged.
+    const uint32_t gw = wave_in_block() * gridDim.x + blockIdx.x, nwaves = gridDim.x * (B / kWave);
+    uint32_t cnt[kPullClasses];
+#pragma unroll
+    for (uint32_t l = 0; l < kPullClasses; ++l) cnt[l] = c->plan[l];
+    const uint32_t nt = c->plan[kPlanTiles];
+    PullAt p0 = pull_at(cnt, gw), p1 = pull_at(cnt, gw + nwaves);
+    PullRows r0, r1;
+    PullQuads q0;
+    pull_load_rows(a, p0, r0);
+    pull_load_rows(a, p1, r1);
+    pull_load_quads(a, p0, r0, q0);
+    if constexpr (HUB) {
+        const uint32_t h = min(a.n, kPullHubs);
+#pragma unroll 8
+        for (uint32_t i = threadIdx.x; i < h; i += B) lds.hub[i] = a.delta[i];
+        __syncthreads();
+    }
+    const PullSrc<HUB> src{a.delta, pass.mask, (LdsFloat *)lds.hub};
     Counters ctr;
-    ctr.vexp = rows_done;
+    uint32_t joined = 0;
+    for (uint32_t u = gw + 2 * nwaves; p0.on; u += nwaves) {
+        const PullAt p2 = pull_at(cnt, u);
+        PullRows r2;
+        PullQuads q1;
+        pull_load_quads(a, p1, r1, q1);
+        pull_load_rows(a, p2, r2);
+        pull_finish(a, src, p0, r0, q0, joined, ctr);
+        p0 = p1;
+        p1 = p2;
+        r0 = r1;
+        r1 = r2;
+        q0 = q1;
+    }
+    if (gw < nt) {
+        Tile next = a.ptiles[gw];
+        for (uint32_t ti = gw; ti < nt; ti += nwaves) {
+            const Tile t = next;
+            if (ti + nwaves < nt) next = a.ptiles[ti + nwaves];
+            pull_tile(a, src, t, ti, joined, ctr);
+        }
+    }
     flush_counters(ctr, a.cfg.stats, pass.stage);
-    out_flush(out);
+    pull_count(c, pass, joined, &total);
 }
 
 // Batch amendment form (Engine::UpdatePageRank, framework.cuh:1660-1704):
@@ -2353,6 +2565,7 @@ __global__ __launch_bounds__(kBlock) void k_ms_consume(MsArgs a, uint64_t *prog,
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         c->qcount[(r + 2) % 3] = 0;
         c->tcount[(r + 2) % 3] = 0;
+        c->fscan[(r + 2) % 3] = c->flist[(r + 2) % 3] = 0;  // a PageRank engine's slots
         if (nq) c->rounds += 1;
         post_progress(prog, tag, nq != 0);
     }
@@ -2391,7 +2604,7 @@ template <int W>
 __global__ __launch_bounds__(kBlock) void k_ms_expand(MsArgs a, uint32_t seq) {
     using Op = decltype(ms_op<W>(a));
     __shared__ PairLds<64 / Op::kGroup> lds[kWavesPerBlock];
-    __shared__ PullStage stage;
+    __shared__ ListStage stage;
     Ctl *c = a.ctl;
     const uint32_t r = c->round + seq - 1;
     const uint32_t nq = c->qcount[r % 3];

@@ -109,7 +109,7 @@ __device__ __forceinline__ unsigned long long msi_bits(const MsiGroup &g, bool f
 // has parent u for source s makes (v, s) affected. Parallel copies of (u,v)
 // are treated conservatively, as in the single-source path.
 __global__ __launch_bounds__(kBlock) void k_msi_inval_seed(MsiArgs a) {
-    __shared__ StageLds<1024, 2> stage;
+    __shared__ ListStage stage;
     const uint32_t r = a.ctl->round;
     const StagedOut<1024, 2> out{Sink{(r & 1) ? a.q1 : a.q0, &a.ctl->qcount[r % 3]}, TileSink{nullptr, &a.ctl->scount},
                                  &stage};
@@ -241,7 +241,7 @@ template <int W, bool INV>
 __global__ __launch_bounds__(kBlock) void k_msi_expand(MsiArgs a, uint32_t seq) {
     using Op = decltype(msi_op<W, INV>(a));
     __shared__ PairLds<64> lds[kWavesPerBlock];
-    __shared__ PullStage stage;
+    __shared__ ListStage stage;
     Ctl *c = a.ctl;
     const uint32_t r = c->round + seq - 1;
     const uint32_t nq = c->qcount[r % 3];
@@ -361,7 +361,7 @@ __global__ __launch_bounds__(kBlock) void k_msi_repair_tiles(MsiArgs a) {
 // After the repair: every affected (y, s) that has a value again is pending
 // expansion, and y joins the frontier of the current round.
 __global__ __launch_bounds__(kBlock) void k_msi_repair_done(MsiArgs a) {
-    __shared__ PullStage stage;
+    __shared__ ListStage stage;
     const uint32_t cnt = ld_acquire(&a.ctl->acount);
     const uint32_t r = a.ctl->round;
     if (threadIdx.x == 0 && blockIdx.x == 0) a.ctl->scount = 0;
@@ -399,7 +399,7 @@ __global__ __launch_bounds__(kBlock) void k_msi_repair_done(MsiArgs a) {
 // affected u re-expands its whole row once repaired).
 template <int W>
 __global__ __launch_bounds__(kBlock) void k_msi_insert_seed(MsiArgs a, uint32_t skip_affected) {
-    __shared__ PullStage stage;
+    __shared__ ListStage stage;
     const uint32_t r = a.ctl->round;
     const StagedOut<1024, 2> out{Sink{(r & 1) ? a.q1 : a.q0, &a.ctl->qcount[r % 3]}, TileSink{nullptr, &a.ctl->scount},
                                  &stage};

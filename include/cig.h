@@ -144,7 +144,8 @@ typedef struct cig_config {
     uint32_t pr_pull_divisor; /* PR rounds whose frontier holds at least n / pr_pull_divisor
                                  vertices gather along the incoming rows instead of scattering
                                  (no atomics); 0 = default (4096); >= n: every round */
-    uint32_t pull_blocks_per_cu; /* workgroups per CU of the PR pull kernels (at most 128); 0 = default (64) */
+    uint32_t pull_blocks_per_cu; /* workgroups per CU of the PR pull kernel (at most 128) where the engine keeps the
+                                    caller's ids; 0 = default (8). A renumbered engine runs one per CU */
     uint32_t kernel_timing_every; /* time one call in this many: its stage markers (the *_ms stage
                                      fields) and, with CIG_CFG_KERNEL_TIMING, its round kernels
                                      (each event record idles the stream a few us); total_ms is
