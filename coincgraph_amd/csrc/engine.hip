@@ -127,17 +127,22 @@ struct HBuf {  // pinned host memory (hipHostMalloc; never hipHostRegister)
     }
 };
 
-// A stream and two pinned bounce buffers that move device results into
-// caller (pageable) memory: the device copies chunk i into one buffer while
-// host threads move chunk i-1 out of the other. The engine's lane uses the
+// A stream and a ring of pinned bounce buffers that move device results into
+// caller (pageable) memory: the device fills the buffers ahead while a team
+// of host threads moves each finished one out (and takes the page faults of a
+// buffer the caller has not touched yet). The runtime's own copy to pageable
+// memory runs at about 10 GB/s here; 16 MB take 0.5 ms this way instead of
+// 1.5, 67 MB 1.6 instead of 6.3. Results below kDirect keep the plain copy,
+// which is done before a team would have started. The engine's lane uses the
 // engine stream; the serving loop has a second lane, so that a query's
 // results leave the device while the next update group runs.
 struct CopyLane {
-    static constexpr uint64_t kChunk = uint64_t(256) << 20;
+    static constexpr uint64_t kChunk = uint64_t(4) << 20, kDirect = uint64_t(2) << 20;
+    static constexpr unsigned kRing = 4, kMovers = 8;
     hipStream_t stream = nullptr;
     bool own_stream = false;
-    HBuf<uint8_t> bounce[2];
-    hipEvent_t ev[2] = {};
+    HBuf<uint8_t> bounce[kRing];
+    hipEvent_t ev[kRing] = {};
     CopyLane() = default;
     CopyLane(const CopyLane &) = delete;
     CopyLane &operator=(const CopyLane &) = delete;
@@ -164,34 +169,66 @@ struct CopyLane {
     }
     // Copies `bytes` from device memory to `out`; returns with the copy complete.
     void copy(void *out, const void *dev, uint64_t bytes) {
-        if (bytes <= kChunk) {
+        if (bytes <= kDirect) {
             HIPCHK(hipMemcpyAsync(out, dev, bytes, hipMemcpyDeviceToHost, stream));
             HIPCHK(hipStreamSynchronize(stream));
             return;
         }
-        if (!bounce[0].p) {
-            for (int b = 0; b < 2; ++b) {
-                bounce[b].alloc(kChunk);
-                HIPCHK(hipEventCreateWithFlags(&ev[b], hipEventDisableTiming));
-            }
+        for (unsigned b = 0; b < kRing; ++b) {
+            if (!bounce[b].p) bounce[b].alloc(kChunk);
+            if (!ev[b]) HIPCHK(hipEventCreateWithFlags(&ev[b], hipEventDisableTiming));
         }
-        const unsigned T = pick_threads(0);
-        auto host_copy = [&](uint64_t chunk) {
-            const uint64_t off = chunk * kChunk, len = std::min(kChunk, bytes - off);
-            HIPCHK(hipEventSynchronize(ev[chunk & 1]));
-            uint8_t *to = static_cast<uint8_t *>(out) + off;
-            const uint8_t *from = bounce[chunk & 1].p;
-            parallel_for(len, T, [&](uint64_t lo, uint64_t hi, unsigned) { std::memcpy(to + lo, from + lo, hi - lo); });
-        };
         const uint64_t chunks = (bytes + kChunk - 1) / kChunk;
-        for (uint64_t i = 0; i < chunks; ++i) {
-            const uint64_t off = i * kChunk, len = std::min(kChunk, bytes - off);
-            HIPCHK(hipMemcpyAsync(bounce[i & 1].p, static_cast<const uint8_t *>(dev) + off, len,
-                                  hipMemcpyDeviceToHost, stream));
-            HIPCHK(hipEventRecord(ev[i & 1], stream));
-            if (i > 0) host_copy(i - 1);  // frees buffer (i-1)&1 for chunk i+1
-        }
-        host_copy(chunks - 1);
+        std::atomic<uint64_t> ready{0};    // chunks in their buffers; ~0: give up
+        std::atomic<unsigned> moved[kRing] = {};  // parts of the buffer's chunk moved out
+        uint64_t issued = 0;
+        auto part = [&](uint64_t c, unsigned t, unsigned movers) {
+            const uint64_t off = c * kChunk, len = std::min(kChunk, bytes - off);
+            const uint64_t step = ((len + movers - 1) / movers + 4095) & ~uint64_t(4095);
+            const uint64_t lo = std::min(len, t * step), hi = std::min(len, lo + step);
+            std::memcpy(static_cast<uint8_t *>(out) + off + lo, bounce[c % kRing].p + lo, hi - lo);
+        };
+        auto issue = [&] {
+            const uint64_t off = issued * kChunk;
+            HIPCHK(hipMemcpyAsync(bounce[issued % kRing].p, static_cast<const uint8_t *>(dev) + off,
+                                  std::min(kChunk, bytes - off), hipMemcpyDeviceToHost, stream));
+            HIPCHK(hipEventRecord(ev[issued % kRing], stream));
+            ++issued;
+        };
+        while (issued < std::min<uint64_t>(kRing, chunks)) issue();
+        std::exception_ptr failed;
+        run_team(std::min(kMovers, pick_threads(0)), [&](unsigned t, unsigned team) {
+            if (t != 0) {
+                for (uint64_t c = 0; c < chunks; ++c) {
+                    uint64_t r;
+                    for (unsigned spin = 0; (r = ready.load(std::memory_order_acquire)) <= c; ++spin)
+                        if (spin > 1024) std::this_thread::yield();
+                    if (r == ~uint64_t(0)) return;
+                    part(c, t, team);
+                    moved[c % kRing].fetch_add(1, std::memory_order_acq_rel);
+                }
+                return;
+            }
+            try {  // the caller's thread drives the device and moves its own parts
+                for (uint64_t c = 0; c < chunks; ++c) {
+                    HIPCHK(hipEventSynchronize(ev[c % kRing]));
+                    ready.store(c + 1, std::memory_order_release);
+                    part(c, 0, team);
+                    moved[c % kRing].fetch_add(1, std::memory_order_acq_rel);
+                    if (c == 0 || issued == chunks) continue;
+                    // the previous chunk's buffer takes the next one, once all its parts have been moved
+                    std::atomic<unsigned> &m = moved[(c - 1) % kRing];
+                    for (unsigned spin = 0; m.load(std::memory_order_acquire) != team; ++spin)
+                        if (spin > 1024) std::this_thread::yield();
+                    m.store(0, std::memory_order_relaxed);
+                    issue();
+                }
+            } catch (...) {
+                failed = std::current_exception();
+                ready.store(~uint64_t(0), std::memory_order_release);
+            }
+        });
+        if (failed) std::rethrow_exception(failed);
     }
 };
 
@@ -3222,17 +3259,15 @@ struct cig_engine {
             }
             return;
         }
+        // a renumbered engine's words go back to the caller's order on the device
         auto words = [&](const uint32_t *src) {
-            if (!renum) {
-                HIPCHK(hipMemcpy(out, src, size_t(n) * 4, hipMemcpyDeviceToHost));
-                return;
+            if (renum) {
+                grow(out_words, n);
+                k_permute_words<<<grid_small, 256, 0, stream>>>(src, perm_d.p, n, out_words.p);
+                HIPCHK(hipGetLastError());
+                src = out_words.p;
             }
-            std::vector<uint32_t> tmp(n);
-            HIPCHK(hipMemcpy(tmp.data(), src, size_t(n) * 4, hipMemcpyDeviceToHost));
-            uint32_t *o = static_cast<uint32_t *>(out);
-            parallel_for(n, pick_threads(0), [&](uint64_t lo, uint64_t hi, unsigned) {
-                for (uint64_t v = lo; v < hi; ++v) o[v] = tmp[perm_h[v]];
-            });
+            copy_out(out, src, uint64_t(n) * 4);
         };
         if (field == CIG_FIELD_HOTNESS) {
             words(score.p);
@@ -3257,11 +3292,12 @@ struct cig_engine {
             copy_out(out, ms_out.p, words * 4);
             return;
         }
-        std::vector<uint64_t> hs(n);
-        HIPCHK(hipMemcpy(hs.data(), state.p, size_t(n) * 8, hipMemcpyDeviceToHost));
-        uint32_t *o = static_cast<uint32_t *>(out);
-        for (uint32_t v = 0; v < n; ++v) o[v] = field == CIG_FIELD_VALUE ? uint32_t(hs[v] >> 32) : uint32_t(hs[v]);
+        grow(out_words, n);
+        k_state_words<<<grid_small, 256, 0, stream>>>(state.p, n, field == CIG_FIELD_VALUE ? 1u : 0u, out_words.p);
+        HIPCHK(hipGetLastError());
+        copy_out(out, out_words.p, uint64_t(n) * 4);
     }
+    DBuf<uint32_t> out_words;  // a result field on its way out (4 B a vertex)
 
     // Rows [first, first+n) as CSR: the outgoing rows (first = 0) or the
     // incoming index (first = n).

@@ -94,3 +94,23 @@ def test_maintained_sources_at_tile_edges(algo, n, k):
             for i in (0, k - 1):
                 res = og.check_parent(exp[i], par[i], int(src[i]), O.W_UNIT if algo == "bfs" else O.W_HASH64, 5)
                 assert res.invalid_vertices == 0, f"batch {b} source {i}"
+
+
+@pytest.mark.parametrize("n", [524287, 524288, 524289, 1048576, 1048577, 4 * 1048576 + 3, 5 * 1048576, 9 * 1048576 + 1])
+def test_result_copy_at_buffer_edges(n):
+    """Results of 4 B a vertex around the direct copy's limit (2 MiB) and the
+    bounce buffers' edges (4 MiB each, a ring of four)."""
+    print(f"[gpu-case] result copy n={n}", flush=True)
+    off = np.zeros(n + 1, dtype=np.uint64)
+    off[n - 1:] = 1
+    g = cg.HostGraph(n, off, np.array([n - 1], dtype=np.uint32))  # one edge, n-2 -> n-1
+    exp = np.arange(n, dtype=np.uint32)
+    par = np.full(n, cg.INF, dtype=np.uint32)
+    exp[n - 1] = par[n - 1] = n - 2
+    with cg.Engine("cc") as e:
+        e.load_graph(g)
+        e.init_graph()
+        e.start()
+        for _ in range(2):
+            assert np.array_equal(e.values(), exp)
+        assert np.array_equal(e.parents(), par)
