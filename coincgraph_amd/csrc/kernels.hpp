@@ -222,8 +222,12 @@ __device__ __forceinline__ const cig_edge *rec_adds(const A &a) { return a.ref ?
 // Deletes find their slot by row length (BuildDeletionPlan,
 // source_local_chunk_store.h:670-723, restated for the device):
 //  - tiny rows (<= 64 slots): one lane per delete record reads the whole row
-//    and claims a matching slot with a CAS (slot := kNone);
-//  - medium rows (<= 4096 slots, <= kDelWaveMax deletes; HBM rows with up to
+//    and claims a matching slot with a CAS (slot := kNone); in the host tier
+//    only those with more than kDelWaveMax deletes: a lane's 16-B reads cross
+//    the host link one by one, a 16-lane group's as whole lines and once per
+//    row (480k delete records of 500,009 vertices with 30% of the edges in
+//    HBM: 4.2 -> 4.0 ms, which is the link's 53 GB/s);
+//  - medium rows (<= 4096 slots, host-tier rows of any length up to that; <= kDelWaveMax deletes; HBM rows with up to
 //    kDelWaveMax16 in a second kernel): a 16-lane group per row against all
 //    of the row's deletes at once, 256 slots a step;
 //  - other rows: tiles of kDelTile slots over the whole grid against the
@@ -265,7 +269,7 @@ constexpr uint64_t kMid16MinRecords = 1u << 20;
 template <bool M16>
 __device__ __forceinline__ uint8_t del_class(uint32_t nd, uint32_t deg, bool host) {
     if (nd == 0) return kDelClassNone;
-    if (deg <= kDelTinyDeg) return kDelClassTiny;
+    if (deg <= kDelTinyDeg && !(host && nd <= kDelWaveMax)) return kDelClassTiny;
     if (deg > kDelMediumDeg) return kDelClassLong;
     if (nd <= kDelWaveMax) return kDelClassMedium;
     return M16 && nd <= kDelWaveMax16 && !host ? kDelClassMedium16 : kDelClassLong;
