@@ -61,8 +61,8 @@ struct Ctl {
     // fixed-point rounds (relax / PR); slot = absolute round % 3
     alignas(kCtlLine) uint32_t qcount[3];
     alignas(kCtlLine) uint32_t tcount[3];
-    uint32_t fscan[3];     // PR: slot's frontier is flags only (a pull pass added to it)
-    alignas(kCtlLine) uint32_t flist[3];   // PR: list entries written by the scan of such a frontier
+    uint32_t fscan[3];     // pull passes (PR, BFS queries): the slot's frontier has no list
+    alignas(kCtlLine) uint32_t flist[3];   // list entries written by the scan of such a frontier
     uint32_t round;        // next absolute round to run
     uint32_t converged;
     alignas(kCtlLine) uint32_t done;  // workgroups finished in the current round kernel

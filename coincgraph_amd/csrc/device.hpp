@@ -918,11 +918,10 @@ __host__ __device__ __forceinline__ uint32_t pair_tile_len(const ExpandCfg &c) {
     return (min(c.tile_len, 2u * c.split) + 3u) & ~3u;
 }
 
-// Cuts this thread's row (when it is long) into tiles; a workgroup-uniform
-// call, one reservation per workgroup.
-__device__ __forceinline__ void pair_cut(const ExpandCfg &cfg, uint32_t v, const Row &row, bool on, Tile *tiles,
-                                         uint32_t *count, uint32_t *scratch) {
-    const uint32_t tl = pair_tile_len(cfg);
+// Cuts this thread's row (when it is long) into tiles of tl slots; a
+// workgroup-uniform call, one reservation per workgroup.
+__device__ __forceinline__ void pair_cut(const ExpandCfg &cfg, uint32_t tl, uint32_t v, const Row &row, bool on,
+                                         Tile *tiles, uint32_t *count, uint32_t *scratch) {
     const uint32_t nt = on && row.deg >= cfg.split ? (row.deg + tl - 1) / tl : 0u;
     const uint32_t at = block_reserve<uint32_t>(nt, count, scratch);
     for (uint32_t j = 0; j < nt; ++j) {

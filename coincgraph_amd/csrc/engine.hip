@@ -247,6 +247,13 @@ constexpr uint32_t kPullDivisorDefault = 4096;
 constexpr uint32_t kPullMaskDivisor = 4;
 constexpr uint32_t kPullMaskMin = 1u << 24;
 constexpr uint32_t kPullBlocksPerCu = 8;
+// BFS queries: rounds whose frontier holds at least n / kMsPullDivisor
+// vertices gather along the incoming rows, in graphs whose rows are all in HBM
+// (a gather reads the rows of every vertex that misses a source, which the
+// host link would pay for). 64 sources of 200,003 vertices, all rounds: n / 4
+// 307 us, n / 16 233, n / 64 252 (a round of n / 40 vertices gathers in 29 us
+// and pushes in 9), never 465.
+constexpr uint32_t kMsPullDivisor = 16;
 
 }  // namespace
 
@@ -3045,6 +3052,12 @@ struct cig_engine {
         a.n = n;
         a.stride = (k + 3u) & ~3u;
         a.seed = cfg.weight_seed;
+        a.all = k == 64 ? ~0ull : (1ull << k) - 1ull;
+        a.pull_min = kNone;
+        if (bfs && pull_rows() && !fl_off.p) {
+            a.in_rows = in_rows_p();
+            a.pull_min = std::max<uint32_t>(1u, n / kMsPullDivisor);
+        }
         SrcList list{};
         std::memcpy(list.v, sources, size_t(k) * 4);
         k_ms_seed<<<1, 64, 0, stream>>>(a, list, k);

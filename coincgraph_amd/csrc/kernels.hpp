@@ -2285,15 +2285,15 @@ __device__ __forceinline__ PullPass pull_pass(const PrArgs &a, uint32_t seq) {
 // not written (flist = 0): a dense consume scans the flags anyway, a sparse
 // one that finds no list scans them too. (A list cost up to an atomic per
 // chunk on one address.) Every thread of the workgroup must call it.
-__device__ __forceinline__ void pull_count(Ctl *c, const PullPass &pass, uint32_t joined, uint32_t *cnt) {
+__device__ __forceinline__ void frontier_count(Ctl *c, uint32_t slot, uint32_t joined, uint32_t *cnt) {
     if (threadIdx.x == 0) *cnt = 0u;
     __syncthreads();
     const uint32_t s = uint32_t(wave_sum64(joined));
     if (s && lane_id() == 0) atomicAdd(cnt, s);
     __syncthreads();
     if (threadIdx.x == 0) {
-        if (*cnt) atomicAdd(&c->qcount[pass.slot], *cnt);
-        if (blockIdx.x == 0) c->fscan[pass.slot] = 1u;
+        if (*cnt) atomicAdd(&c->qcount[slot], *cnt);
+        if (blockIdx.x == 0) c->fscan[slot] = 1u;
     }
 }
 
@@ -2379,7 +2379,7 @@ __global__ __launch_bounds__(HUB ? kPullHubBlock : kBlock) void k_pr_pull(PrArgs
         }
     }
     flush_counters(ctr, a.cfg.stats, pass.stage);
-    pull_count(c, pass, joined, &total);
+    frontier_count(c, pass.slot, joined, &total);
 }
 
 // Batch amendment form (Engine::UpdatePageRank, framework.cuh:1660-1704):
@@ -2440,7 +2440,14 @@ struct MsArgs {
     ExpandCfg cfg;
     uint32_t n, stride;
     uint64_t seed;
+    // BFS pull rounds: incoming rows (null: push only), the frontier size from
+    // which a round gathers, the run's source bits
+    const Row *in_rows;
+    uint32_t pull_min;
+    unsigned long long all;
 };
+
+__device__ __forceinline__ bool ms_dense(const MsArgs &a, uint32_t nq) { return nq != 0 && nq >= a.pull_min; }
 
 // A group is four sources: one 16-B load of the row owner's distances and one
 // of the destination's.
@@ -2559,67 +2566,210 @@ __device__ __forceinline__ void ms_write_depths(uint32_t *dist, uint32_t stride,
 
 // Round round+seq-1, phase 1: snapshot and clear the masks of the frontier,
 // cut its long rows into tiles (so that phase 2 expands rows and tiles of one
-// round in one launch); BFS: write the depths of the bits taken.
+// round in one launch); BFS: write the depths of the bits taken. A dense BFS
+// round (ms_dense) walks every vertex instead of the list: its pull needs a
+// snapshot of each (0 outside the frontier) and cuts the long incoming rows
+// of the vertices that still miss sources. A frontier that a pull left
+// without a list (fscan) is found the same way.
 template <bool BFS>
 __global__ __launch_bounds__(kBlock) void k_ms_consume(MsArgs a, uint64_t *prog, uint64_t tag, uint32_t seq) {
     __shared__ uint32_t scratch[kMaxWavesPerBlock + 1];
     Ctl *c = a.ctl;
     const uint32_t r = c->round + seq - 1;
     const uint32_t nq = c->qcount[r % 3];
+    const bool dense = BFS && ms_dense(a, nq), scan = BFS && nq != 0 && (dense || c->fscan[r % 3] != 0);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         c->qcount[(r + 2) % 3] = 0;
         c->tcount[(r + 2) % 3] = 0;
-        c->fscan[(r + 2) % 3] = c->flist[(r + 2) % 3] = 0;  // a PageRank engine's slots
+        c->fscan[(r + 2) % 3] = c->flist[(r + 2) % 3] = 0;
         if (nq) c->rounds += 1;
         post_progress(prog, tag, nq != 0);
     }
-    const uint32_t *qin = (r & 1) ? a.q1 : a.q0;
+    uint32_t *qin = (r & 1) ? a.q1 : a.q0;
+    const uint32_t bound = scan ? a.n : nq;
     Counters ctr;
-    for (uint32_t base = blockIdx.x * blockDim.x; base < nq; base += gthreads()) {
+    for (uint32_t base = blockIdx.x * blockDim.x; base < bound; base += gthreads()) {
         const uint32_t i = base + threadIdx.x;
-        const bool on = i < nq;
+        bool on = i < bound;
         uint32_t v = 0;
         Row row{};
         unsigned long long m = 0;
         if (on) {
-            v = qin[i];
-            row = a.rows[v];
+            v = scan ? i : qin[i];
             if constexpr (BFS) {
                 const ulonglong2 x = *reinterpret_cast<const ulonglong2 *>(a.reach + 2ull * v);
                 m = x.x & ~x.y;
-                a.reach[2ull * v + 1] = x.x;
+                if (m) a.reach[2ull * v + 1] = x.x;
+                if (dense) {
+                    a.snap[v] = m;
+                    on = (a.all & ~x.x) != 0ull;  // this vertex gathers
+                    if (on) row = a.in_rows[v];
+                } else {
+                    on = m != 0ull;
+                }
             } else {
                 m = a.act[v];
                 a.act[v] = 0ull;
             }
-            a.snap[v] = m;
-            ctr.scanned += row.deg;
-            ctr.vexp += row.deg ? 1 : 0;
-            if (row.off & kHostTier) ctr.host += row.deg;
+            if (on && !dense) {
+                row = a.rows[v];
+                a.snap[v] = m;
+            }
+            if (on) {
+                ctr.scanned += row.deg;
+                ctr.vexp += row.deg ? 1 : 0;
+                if (row.off & kHostTier) ctr.host += row.deg;
+            }
         }
-        pair_cut(a.cfg, v, row, on, a.tiles, &c->tcount[r % 3], scratch);
+        if constexpr (BFS) {
+            if (scan && !dense) {  // the list the expansion reads
+                const uint32_t at = block_reserve<uint32_t>(on ? 1u : 0u, &c->flist[r % 3], scratch);
+                if (on) qin[at] = v;
+            }
+        }
+        pair_cut(a.cfg, dense ? a.cfg.tile_len : pair_tile_len(a.cfg), v, row, on, a.tiles, &c->tcount[r % 3], scratch);
         if constexpr (BFS) ms_write_depths(a.dist, a.stride, v, m, seq - 1);
     }
     if (nq) flush_counters(ctr, a.cfg.stats, a.cfg.stage);
 }
 
-// Phase 2: expand the frontier's rows and tiles.
+// BFS pull: the sources that reach v in this round are the OR of its
+// in-neighbours' snapshots, so a vertex is written once, by its own lane. In
+// a dense push every edge into a hub that has not seen the hub's new bits yet
+// queues an atomicOr at the hub (64 sources of 200,003 vertices: rounds of
+// 125, 160, 95 and 36 us pushed, 46, 46, 46 and 42 gathered). Bound by the
+// gathers, each of which moves a 128-B line into L1 for one snapshot: 3 M
+// edges a round, 9 TB/s. 16, 32 and 64 vertices a wave: 50, 46 and 50 us.
+constexpr uint32_t kPullVertices = 32;
+struct MsPullLds {
+    uint32_t pref[kWave], offlo[kWave], offhi[kWave];
+    unsigned long long acc[kWave];
+};
+
+// The kPullVertices vertices from v0: those that miss sources and have a short row.
+__device__ void ms_pull_chunk(const MsArgs &a, uint32_t v0, MsPullLds &L, uint32_t &joined) {
+    constexpr uint32_t U = 4;
+    const uint32_t lane = lane_id(), v = v0 + lane;
+    unsigned long long missing = 0;
+    uint32_t deg = 0;
+    uint64_t off = 0;
+    if (lane < kPullVertices && v < a.n) {
+        const Row row = a.in_rows[v];  // with the mask's load, not behind it
+        missing = a.all & ~a.reach[2ull * v];
+        deg = missing && row.deg < a.cfg.split ? row.deg : 0u;
+        off = row.off;
+    }
+    const uint32_t incl = wave_incl_scan(deg);
+    const uint32_t total = __shfl(incl, kWave - 1, kWave);
+    if (total == 0) return;
+    L.pref[lane] = incl - deg;
+    L.offlo[lane] = uint32_t(off);
+    L.offhi[lane] = uint32_t(off >> 32);
+    L.acc[lane] = 0ull;
+    wave_lds_sync();
+    for (uint32_t k0 = 0; k0 < total; k0 += kWave * U) {
+        uint32_t own[U], rest[U], w[U];
+        unsigned long long x[U];
+        bool head[U];
+#pragma unroll
+        for (uint32_t i = 0; i < U; ++i) {
+            const uint32_t k = k0 + i * kWave + lane, kk = k < total ? k : total - 1;
+            own[i] = owner_of(L.pref, kk);
+            const uint32_t at = kk - L.pref[own[i]];
+            const uint32_t end = own[i] + 1 < uint32_t(kWave) ? L.pref[own[i] + 1] : total;
+            w[i] = a.cfg.pools.row((uint64_t(L.offhi[own[i]]) << 32) | L.offlo[own[i]])[at];
+            rest[i] = min(end - 1u - kk, uint32_t(kWave) - 1u - lane);
+            head[i] = k < total && (at == 0 || lane == 0);
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < U; ++i) x[i] = a.snap[w[i]];
+#pragma unroll
+        for (uint32_t i = 0; i < U; ++i) {
+            if (__ballot(x[i] != 0ull) == 0) continue;
+#pragma unroll
+            for (uint32_t d = 1; d < uint32_t(kWave); d <<= 1) {
+                const unsigned long long y = __shfl_down(x[i], d, kWave);
+                if (d <= rest[i]) x[i] |= y;
+            }
+            if (head[i]) L.acc[own[i]] |= x[i];
+            wave_lds_sync();
+        }
+    }
+    wave_lds_sync();
+    const unsigned long long gained = deg ? L.acc[lane] & missing : 0ull;
+    if (gained) {
+        a.reach[2ull * v] |= gained;
+        ++joined;
+    }
+    wave_lds_sync();  // LDS is reused by the next chunk of this wave
+}
+
+// One tile of a long incoming row: one atomic per tile that adds sources.
+__device__ void ms_pull_tile(const MsArgs &a, const Tile &t, uint32_t &joined) {
+    constexpr uint32_t U = 8;
+    const uint32_t lane = lane_id();
+    const ulonglong2 cur = *reinterpret_cast<const ulonglong2 *>(a.reach + 2ull * t.v);
+    const unsigned long long missing = a.all & ~cur.x;
+    if (missing == 0ull) return;
+    const uint32_t *p = a.cfg.pools.row(t.start);
+    unsigned long long acc = 0;
+    for (uint32_t k0 = 0; k0 < t.len; k0 += kWave * U) {
+        uint32_t w[U];
+        unsigned long long x[U];
+#pragma unroll
+        for (uint32_t i = 0; i < U; ++i) w[i] = p[min(k0 + i * kWave + lane, t.len - 1)];
+#pragma unroll
+        for (uint32_t i = 0; i < U; ++i) x[i] = a.snap[w[i]];
+#pragma unroll
+        for (uint32_t i = 0; i < U; ++i) acc |= x[i];
+    }
+#pragma unroll
+    for (int d = kWave / 2; d > 0; d >>= 1) acc |= __shfl_xor(acc, d, kWave);
+    if (lane != 0 || (acc & missing) == 0ull) return;
+    // the first tile to add sources this round finds seen and done equal
+    const unsigned long long old = atomicOr(&a.reach[2ull * t.v], acc & missing);
+    if (old == cur.y && (acc & missing & ~old)) ++joined;
+}
+
+// Phase 2: expand the frontier's rows and tiles, or gather (a dense BFS round).
 template <int W>
 __global__ __launch_bounds__(kBlock) void k_ms_expand(MsArgs a, uint32_t seq) {
     using Op = decltype(ms_op<W>(a));
-    __shared__ PairLds<64 / Op::kGroup> lds[kWavesPerBlock];
-    __shared__ ListStage stage;
+    struct Push {
+        PairLds<64 / Op::kGroup> pair[kWavesPerBlock];
+        ListStage stage;
+    };
+    union Lds {
+        Push push;
+        MsPullLds pull[W == 2 ? kWavesPerBlock : 1];
+        __device__ Lds() {}
+    };
+    __shared__ Lds lds;
     Ctl *c = a.ctl;
     const uint32_t r = c->round + seq - 1;
     const uint32_t nq = c->qcount[r % 3];
     if (nq == 0) return;
+    const uint32_t nt = c->tcount[r % 3];
+    if constexpr (W == 2) {
+        if (ms_dense(a, nq)) {
+            __shared__ uint32_t total;
+            uint32_t joined = 0;
+            const uint32_t gw = wave_in_block() * gridDim.x + blockIdx.x, nw = gwaves();
+            for (uint32_t t = gw; t < nt; t += nw) ms_pull_tile(a, a.tiles[t], joined);
+            const uint32_t chunks = (a.n + kPullVertices - 1) / kPullVertices;
+            for (uint32_t ch = gw; ch < chunks; ch += nw)
+                ms_pull_chunk(a, ch * kPullVertices, lds.pull[wave_in_block()], joined);
+            frontier_count(c, (r + 1) % 3, joined, &total);
+            return;
+        }
+    }
     const Op op = ms_op<W>(a);
     const StagedOut<1024, 2> out{Sink{(r & 1) ? a.q0 : a.q1, &c->qcount[(r + 1) % 3]}, TileSink{nullptr, &c->scount},
-                                 &stage};
+                                 &lds.push.stage};
     out_init(out);
-    PairLds<64 / Op::kGroup> &L = lds[wave_in_block()];
+    PairLds<64 / Op::kGroup> &L = lds.push.pair[wave_in_block()];
     pair_range<Op::kGroup, Op::kUnroll>(op, a.cfg, a.rows, (r & 1) ? a.q1 : a.q0, nq, L, out);
-    pair_tiles<Op::kGroup, Op::kUnroll>(op, a.cfg, a.tiles, c->tcount[r % 3], L, out);
+    pair_tiles<Op::kGroup, Op::kUnroll>(op, a.cfg, a.tiles, nt, L, out);
     out_flush(out);
 }
 

@@ -224,7 +224,7 @@ __global__ __launch_bounds__(kBlock) void k_msi_consume(MsiArgs a, unsigned long
             ctr.vexp += row.deg ? 1 : 0;
             if (row.off & kHostTier) ctr.host += row.deg;
         }
-        pair_cut(a.cfg, v, row, on, a.tiles, &c->tcount[r % 3], scratch);
+        pair_cut(a.cfg, pair_tile_len(a.cfg), v, row, on, a.tiles, &c->tcount[r % 3], scratch);
     }
     if (nq) flush_counters(ctr, a.cfg.stats, a.cfg.stage);
 }
@@ -323,7 +323,7 @@ __global__ __launch_bounds__(kBlock) void k_msi_repair(MsiArgs a) {
             ctr.vexp += row.deg ? 1 : 0;
             if (row.off & kHostTier) ctr.host += row.deg;
         }
-        pair_cut(a.cfg, y, row, i < na, a.tiles, &c->scount, scratch);
+        pair_cut(a.cfg, pair_tile_len(a.cfg), y, row, i < na, a.tiles, &c->scount, scratch);
     }
     flush_counters(ctr, a.cfg.stats, a.cfg.stage);
     const MsiPullOp<W> op{a.st, a.affm, nullptr, a.k, a.seed};
