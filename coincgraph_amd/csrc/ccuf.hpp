@@ -30,6 +30,7 @@ struct UfArgs {
     uint32_t na;
     const uint8_t *add_skip, *del_skip;
     uint32_t n;
+    uint32_t ts;  // stage markers the kernel notes
 };
 
 __device__ __forceinline__ uint32_t uf_load(const uint32_t *p) {
@@ -63,6 +64,7 @@ __device__ __forceinline__ void uf_unite(uint32_t *uf, uint32_t a, uint32_t b) {
 // derived like a deleted-into component).
 __global__ void k_uf_init(UfArgs a) {
     __shared__ uint32_t scratch[kMaxWavesPerBlock + 1];
+    stamp_marks(a.ctl, a.ts);
     for (uint32_t base = blockIdx.x * blockDim.x; base < a.n; base += gthreads()) {
         const uint32_t v = base + threadIdx.x;
         if (v < a.n) a.uf[v] = v;
@@ -73,6 +75,7 @@ __global__ void k_uf_init(UfArgs a) {
 // The labels of the components the deletes touch (both endpoints of an
 // undirected edge carry the same label).
 __global__ void k_uf_mark(UfArgs a) {
+    stamp_marks(a.ctl, a.ts);
     for (uint32_t i = gthread(); i < a.nd; i += gthreads()) {
         const cig_edge e = a.dels[i];
         if (e.u >= a.n || e.v >= a.n || (a.del_skip && a.del_skip[i])) continue;
@@ -170,6 +173,7 @@ __global__ __launch_bounds__(kBlock) void k_uf_hook(UfArgs a) {
     __shared__ WaveLds lds[kWavesPerBlock];
     __shared__ StageLds<2, 128> stage;
     Ctl *c = a.ctl;
+    stamp_marks(c, a.ts);
     const uint32_t cnt = ld_acquire(&c->acount);
     if (cnt == 0) return;
     const UfHookOp op{a.rows, a.uf, a.roots, c->ufsel[0]};
@@ -184,6 +188,7 @@ __global__ __launch_bounds__(kBlock) void k_uf_hook(UfArgs a) {
 template <int QPL>
 __global__ __launch_bounds__(kBlock) void k_uf_hook_tiles(UfArgs a) {
     Ctl *c = a.ctl;
+    stamp_marks(c, a.ts);
     const uint32_t nt = ld_acquire(&c->scount);
     if (nt == 0) return;
     const UfHookOp op{a.rows, a.uf, a.roots, c->ufsel[0]};
@@ -207,6 +212,7 @@ __global__ void k_uf_flatten(UfArgs a) {
 
 // Inserted edges unite their components.
 __global__ void k_uf_union_adds(UfArgs a) {
+    stamp_marks(a.ctl, a.ts);
     for (uint32_t i = gthread(); i < a.na; i += gthreads()) {
         const cig_edge e = a.adds[i];
         if (e.u >= a.n || e.v >= a.n || (a.add_skip && a.add_skip[i])) continue;

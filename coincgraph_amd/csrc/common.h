@@ -109,6 +109,10 @@ struct Ctl {
     uint64_t touched_sources;
     uint64_t rounds;
     double residual_l1;
+    // stage markers: device clock ticks (see stamp_marks); 0 call start,
+    // 1 mutated, 2 invalidated, 3 repaired, 5 seeded, 4 propagated, 6 group
+    // start, 7 call end, 8/9 around the repair kernel
+    uint64_t ts[10];
     // per expansion pass: 0 invalidation, 1 repair scan, 2 propagation, 3 PR amend
     uint64_t st_edges[4];
     uint64_t st_vexp[4];

@@ -264,7 +264,7 @@ struct cig_engine {
     int device = 0;
     int cus = 0;
     hipStream_t stream = nullptr;
-    hipEvent_t ev[10] = {};
+    double tick_ms = 0.0;  // of the device's constant-rate clock (stage markers)
     // A second compute stream: a batch's invalidation waves run on it while
     // the engine stream groups the batch's records (see traversal_batch).
     hipStream_t side = nullptr;
@@ -278,7 +278,7 @@ struct cig_engine {
     bool side_pending = false, side_ready = false;
     bool fresh_records = false;  // this call enqueued nothing before its batch (resident records)
     bool overlapped = false;  // this call's invalidation ran beside the grouping
-    bool scan_timed = false;  // ev[8]/ev[9] bracket this call's repair scan kernel
+    bool scan_timed = false;  // markers 8 and 9 bracket this call's repair scan kernel
     // CIG_CFG_KERNEL_TIMING: an event pair per propagation round launch
     static constexpr uint32_t kRoundEvents = 512;
     std::vector<hipEvent_t> rev_begin, rev_end;
@@ -409,7 +409,9 @@ struct cig_engine {
         HIPCHK(hipEventCreateWithFlags(&side_done_ev, hipEventDisableTiming));
         scratch_dev = scratch_address(cfg.device);
         lane.init(stream);
-        for (auto &e : ev) HIPCHK(hipEventCreate(&e));
+        int khz = 0;
+        HIPCHK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, cfg.device));
+        tick_ms = 1.0 / double(std::max(1, khz));
         if (cfg.flags & CIG_CFG_KERNEL_TIMING) {
             rev_begin.resize(kRoundEvents);
             rev_end.resize(kRoundEvents);
@@ -877,8 +879,10 @@ struct cig_engine {
         sync();
     }
 
-    void reset_ctl(bool keep_rounds, bool keep_mut = false) {
-        k_reset_ctl<<<1, 64, 0, stream>>>(ctl.p, (keep_rounds ? kResetKeepRounds : 0u) | (keep_mut ? kResetKeepMut : 0u));
+    void reset_ctl(bool keep_rounds, bool keep_mut = false, bool call_start = false) {
+        if (!keep_rounds) rounds_pending = 0;
+        k_reset_ctl<<<1, 64, 0, stream>>>(ctl.p, (keep_rounds ? kResetKeepRounds : 0u) |
+                                                     (keep_mut ? kResetKeepMut : 0u) | (call_start ? kResetStamp : 0u));
         HIPCHK(hipGetLastError());
     }
 
@@ -959,11 +963,28 @@ struct cig_engine {
     bool timing_now = false;      // this call's round kernels are timed
     bool stages_now = true;       // this call records its stage markers
 
-    // Stage marker k (ev[k]) of a sampled call. Each event record costs the
-    // stream a few microseconds of idle, so calls that kernel_timing_every
-    // skips record only their begin/end pair.
+    // Stage marker k (Ctl::ts) of a sampled call: noted by the next kernel
+    // that takes pending markers (take_marks), at the latest by the one that
+    // ends the call. mark_now: by a small kernel of its own, where the next
+    // one takes none.
+    uint32_t marks_pending = 0;
     void mark(int k) {
-        if (stages_now) HIPCHK(hipEventRecord(ev[k], stream));
+        if (stages_now) marks_pending |= 1u << k;
+    }
+    void mark_always(int k) { marks_pending |= 1u << k; }  // markers of every call
+    uint32_t take_marks() {
+        const uint32_t m = marks_pending;
+        marks_pending = 0;
+        return m;
+    }
+    void flush_marks() {
+        if (!marks_pending) return;
+        k_mark<<<1, 64, 0, stream>>>(ctl.p, take_marks());
+        HIPCHK(hipGetLastError());
+    }
+    void mark_now(int k) {
+        mark(k);
+        flush_marks();
     }
 
     // Launches one propagation round kernel, bracketed by an event pair when
@@ -979,8 +1000,16 @@ struct cig_engine {
         }
     }
 
+    // The chain that ends a call leaves its advance to the kernel that ends
+    // the call (k_end_call): nothing in between reads the round counter.
+    bool last_chain = false;
+    uint32_t rounds_pending = 0;
     void advance_round(uint64_t by) {
         if (!by) return;
+        if (last_chain) {
+            rounds_pending += uint32_t(by);
+            return;
+        }
         k_advance_round<<<1, 64, 0, stream>>>(ctl.p, uint32_t(by));
         HIPCHK(hipGetLastError());
     }
@@ -1001,6 +1030,7 @@ struct cig_engine {
             // deferred tile), so a larger count means a broken invariant.
             const uint32_t cap = cfg.max_rounds ? cfg.max_rounds : round_bound();
             LoopArgs a = loop_args(cap);
+            flush_marks();
             launch_coop(kernel, a, grid);
             if (cfg.max_rounds) {
                 for (uint32_t i = 0; i < launches_cap; ++i) {
@@ -1012,6 +1042,7 @@ struct cig_engine {
         } else if (ordered()) {
             LoopArgs a = loop_args(1);
             const uint64_t bound = cfg.max_rounds ? cfg.max_rounds : round_bound();
+            flush_marks();
             k_ord_reset<<<1, 64, 0, stream>>>(ctl.p);
             advance_round(run_chain(
                 [&](uint64_t tag, uint32_t seq) {
@@ -1023,6 +1054,7 @@ struct cig_engine {
                 bound, "ordered relax fixed point"));
         } else {
             LoopArgs a = loop_args(1);
+            a.ts = take_marks();
             const uint64_t bound = cfg.max_rounds ? cfg.max_rounds : round_bound();
             advance_round(run_chain(
                 [&](uint64_t tag, uint32_t seq) {
@@ -1048,7 +1080,9 @@ struct cig_engine {
         }
     }
 
-    void relax() {
+    // last: the chain that ends the call (see advance_round)
+    void relax(bool last = false) {
+        last_chain = last;
         switch (qpl) {
         case 1: relax_dispatch_qpl<1>(); break;
         case 4: relax_dispatch_qpl<4>(); break;
@@ -1114,6 +1148,8 @@ struct cig_engine {
     // current incoming rows.
     void pr_converge(bool plan_ready = false) {
         if (pull_rows() && !coop) ensure_pull();
+        flush_marks();
+        last_chain = true;
         PrArgs a = pr_args(cfg.pr_max_rounds);
         if (coop) {
             auto kernel = k_pr_loop<1>;
@@ -1180,13 +1216,19 @@ struct cig_engine {
     }
 
     // ------------------------------------------------------------ stats
-    // quick: an overlapped call whose side stream is ready (side_ready): the
-    // start event comes first, nothing waits for the side stream and the
-    // mutation counters are left to it.
+    // quick: an overlapped call whose side stream is ready (side_ready):
+    // nothing waits for the side stream and the mutation counters are left to
+    // it.
     void begin_call(cig_batch_stats *st, bool quick = false) {
         if (st) std::memset(st, 0, sizeof(*st));
-        if (quick) HIPCHK(hipEventRecord(ev[0], stream));
-        else flush_finish();
+        marks_pending = 0;
+        last_chain = false;
+        if (rounds_pending) {  // a call that ended by an exception
+            const uint32_t by = rounds_pending;
+            rounds_pending = 0;
+            advance_round(by);
+        }
+        if (!quick) flush_finish();
         scan_timed = false;
         overlapped = false;
         round_timed = 0;
@@ -1196,8 +1238,7 @@ struct cig_engine {
         stages_now = calls % every == 0;
         timing_now = !rev_begin.empty() && stages_now;
         ++calls;
-        reset_ctl(true, quick);
-        if (!quick) HIPCHK(hipEventRecord(ev[0], stream));
+        reset_ctl(true, quick, true);  // notes marker 0
     }
 
     // Time between two recorded events. A call that ends by polling its
@@ -1212,11 +1253,8 @@ struct cig_engine {
         HIPCHK(r);
     }
 
-    float elapsed(int a, int b) {
-        float ms = 0;
-        event_ms(ev[a], ev[b], &ms);
-        return ms;
-    }
+    // Milliseconds between two markers of the control block read last.
+    double elapsed(int a, int b) const { return double(int64_t(hctl.p->ts[b] - hctl.p->ts[a])) * tick_ms; }
 
     void reduce_stats() {
         k_reduce_stats<<<1, kWave, 0, stream>>>(stats.p, ctl.p);
@@ -1228,9 +1266,12 @@ struct cig_engine {
     // (a copy plus a stream synchronisation costs tens of microseconds of
     // wake-up between consecutive calls). When it returns, all of the call's
     // work on the engine stream is done.
-    void read_ctl_published() {
+    void end_and_read_ctl() {
         const uint64_t seq = ++pub_seq;
-        k_publish_ctl<<<1, 64, 0, stream>>>(ctl.p, pub_dev, seq);
+        mark_always(7);
+        k_end_call<<<1, kWave, 0, stream>>>(ctl.p, stats.p, pub_dev, seq, rounds_pending, take_marks());
+        rounds_pending = 0;
+        last_chain = false;
         HIPCHK(hipGetLastError());
         for (uint32_t spin = 0;; ++spin) {
             if (__atomic_load_n(&pub.p->seq, __ATOMIC_ACQUIRE) == seq) break;
@@ -1247,9 +1288,7 @@ struct cig_engine {
     }
 
     void end_call(cig_batch_stats *st, int marks) {
-        HIPCHK(hipEventRecord(ev[7], stream));
-        reduce_stats();
-        read_ctl_published();
+        end_and_read_ctl();
         if (hctl.p->pr_invalid) throw HipError(CIG_EINTERNAL, "PR non-finite rank/residual");
         if (!is_pr() && !cfg.max_rounds) {
             const uint32_t r = hctl.p->round;
@@ -1259,7 +1298,7 @@ struct cig_engine {
         if (!st) return;
         const Ctl &c = *hctl.p;
         st->total_ms = elapsed(0, 7);
-        if (marks >= 4 && stages_now) {  // ev: 0 start, 1 mutated, 2 invalidated, 3 repaired, 5 seeded, 4 propagated
+        if (marks >= 4 && stages_now) {
             st->mutate_ms = elapsed(0, 1);
             // overlapped: the invalidation ran beside the mutation, from the start
             st->invalidate_ms = overlapped ? elapsed(0, 2) : elapsed(1, 2);
@@ -1378,9 +1417,11 @@ struct cig_engine {
 
     // claimed: mutate_claims ran already (the second stream of an overlapped
     // batch); then only the hole fixes and the adds are left.
-    void mutate_apply(const MutArgs &m, bool claimed = false) {
+    void mutate_apply(const MutArgs &ma, bool claimed = false) {
+        MutArgs m = ma;
         if (m.nd) {
             if (!claimed) mutate_claims(m);
+            m.ts = m.ref ? 0u : take_marks();  // (a captured launch takes none)
             k_del_fix_both<<<grid_small, 256, 0, stream>>>(m, grid_small / 2);
         }
         k_add_plan<<<grid_small, 256, 0, stream>>>(m, add_list.p, &ctl.p->add_cnt);
@@ -1867,13 +1908,14 @@ struct cig_engine {
     void repair_scan_qpl(const InvalArgs &ia) {
         InvalArgs a = ia;
         a.cfg = ecfg(kStageRepair);
+        flush_marks();
         fill32(filt.p, kFilterWords, 0);
         k_build_filter<<<grid_small, 256, 0, stream>>>(a);
         // 32 KB filter + 8 wave slots of LDS per workgroup: 3 workgroups per CU
         const uint32_t grid = uint32_t(cus) * 3;
-        mark(8);
+        mark_now(8);
         k_repair_scan<W, S, QPL><<<grid, kRepairBlock, 0, stream>>>(a);
-        mark(9);
+        mark_now(9);
         scan_timed = stages_now;
         k_repair_tiles<W, S, QPL><<<grid, kRepairBlock, 0, stream>>>(a);
         HIPCHK(hipGetLastError());
@@ -1893,8 +1935,10 @@ struct cig_engine {
         InvalArgs a = ia;
         a.cfg = ecfg(kStageRepair);
         mark(8);
+        a.ts = take_marks();
         k_repair_pull<W, S, QPL><<<grid_small, kBlock, 0, stream>>>(a);
         mark(9);
+        a.ts = take_marks();
         scan_timed = stages_now;
         k_repair_pull_tiles<W, S, QPL><<<grid_small, kBlock, 0, stream>>>(a);
         HIPCHK(hipGetLastError());
@@ -1914,15 +1958,18 @@ struct cig_engine {
 
     template <int W, bool S>
     void insert_seed(const InvalArgs &ia, bool skip_affected) {
-        k_insert_seed<W, S><<<grid_small, 256, 0, stream>>>(ia, skip_affected ? 1u : 0u);
+        InvalArgs a = ia;
+        a.ts = take_marks();
+        k_insert_seed<W, S><<<grid_small, 256, 0, stream>>>(a, skip_affected ? 1u : 0u);
         HIPCHK(hipGetLastError());
     }
 
     void invalidate_and_reset(const InvalArgs &ia, hipStream_t on = nullptr, bool reset = true) {
         if (!on) on = stream;
-        k_inval_seed<<<ia.ref ? grid_small : grid_for(ia.nd, 1), 256, 0, on>>>(ia);
-        HIPCHK(hipGetLastError());
         InvalArgs a = ia;
+        a.ts = take_marks();
+        k_inval_seed<<<ia.ref ? grid_small : grid_for(ia.nd, 1), 256, 0, on>>>(a);
+        HIPCHK(hipGetLastError());
         if (coop) {
             auto kernel = k_inval_loop<1>;
             static thread_local uint32_t grid = 0;
@@ -2072,7 +2119,7 @@ struct cig_engine {
                 (void)hipStreamSynchronize(side);
                 throw;
             }
-            mark(2);
+            mark_now(2);  // (captured launches take no markers)
             HIPCHK(hipStreamWaitEvent(stream, join_ev, 0));
             graph_run(graph_apply, sig, [&] {
                 switch (qpl) {
@@ -2086,14 +2133,14 @@ struct cig_engine {
             mark(1);
             mark(3);
             mark(5);
-            relax();
+            relax(true);
             mark(4);
             end_call(st, 4);
             if (na && hctl.p->overflow_cnt) {
                 recover_overflow(m);
                 ia.ref = bref.p;
                 insert_seed<W, S>(ia, false);
-                relax();
+                relax(true);
                 end_call(st, 4);
             }
             finish_split(m);
@@ -2105,14 +2152,14 @@ struct cig_engine {
             k_inval_seed<<<grid_small, 256, 0, stream>>>(ic);
             HIPCHK(hipGetLastError());
         });
-        mark(1);
+        mark_now(1);
         if (nd) {
             inval_waves += run_chain([&](uint64_t tag, uint32_t seq) {
                           k_inval_round<1><<<grid_round, kBlock, 0, stream>>>(ia, prog_dev, tag, seq);
                       },
                       round_bound(), "invalidation");
         }
-        mark(2);
+        mark_now(2);
         graph_run(graph_repair, sig, [&] {
             switch (qpl) {
             case 1: graph_repair_body<W, S, 1>(ic); break;
@@ -2122,14 +2169,14 @@ struct cig_engine {
         });
         mark(3);
         mark(5);
-        relax();
+        relax(true);
         mark(4);
         end_call(st, 4);
         if (na && hctl.p->overflow_cnt) {
             recover_overflow(m);
             ia.ref = bref.p;
             insert_seed<W, S>(ia, false);
-            relax();
+            relax(true);
             end_call(st, 4);
         }
         defer_finish(m, nd != 0);
@@ -2204,7 +2251,7 @@ struct cig_engine {
         mark(3);
         if (na) insert_seed<W, S>(ia, nd != 0);
         mark(5);
-        relax();
+        relax(true);
         mark(4);
         // One host read per batch: end_call's control-block read also tells
         // whether any insert found no room (then recover, re-seed those
@@ -2213,7 +2260,7 @@ struct cig_engine {
         if (na && hctl.p->overflow_cnt) {
             recover_overflow(m);
             insert_seed<W, S>(ia, false);
-            relax();
+            relax(true);
             end_call(st, 4);  // the control block still holds the whole call's totals
         }
         if (overlap) finish_split(m);
@@ -2301,13 +2348,16 @@ struct cig_engine {
 
     // Sample, snapshot, select, hook and flatten the listed vertices.
     template <int QPL>
-    void uf_derive_qpl(const UfArgs &x) {
+    void uf_derive_qpl(const UfArgs &xa) {
+        UfArgs x = xa;
         k_uf_sample<<<grid_small, 256, 0, stream>>>(x);
         k_uf_snapshot<<<grid_small, 256, 0, stream>>>(x);
         k_uf_select<<<1, 256, 0, stream>>>(x);
         mark(8);
+        x.ts = take_marks();
         k_uf_hook<QPL><<<grid_small, kBlock, 0, stream>>>(x);
         mark(9);
+        x.ts = take_marks();
         scan_timed = stages_now;
         k_uf_hook_tiles<QPL><<<grid_small, kBlock, 0, stream>>>(x);
         k_uf_flatten<<<grid_small, 256, 0, stream>>>(x);
@@ -2326,6 +2376,7 @@ struct cig_engine {
     void uf_all() {
         reset_ctl(false);  // drops the label-propagation frontier cig_init left
         UfArgs x = uf_args(nullptr, 0, nullptr, 0);
+        x.ts = take_marks();
         k_uf_init<<<grid_small, 256, 0, stream>>>(x);
         uf_derive(x);
     }
@@ -2336,8 +2387,9 @@ struct cig_engine {
         mutate_group(m);
         mutate_apply(m);
         mark(1);
-        const UfArgs x = uf_args(d, nd, a, na);
+        UfArgs x = uf_args(d, nd, a, na);
         if (nd) {
+            x.ts = take_marks();
             k_uf_mark<<<grid_small, 256, 0, stream>>>(x);
             k_uf_collect<<<grid_small, 256, 0, stream>>>(x);
             uf_derive(x);
@@ -2345,6 +2397,7 @@ struct cig_engine {
         mark(2);
         mark(3);
         if (na) {
+            x.ts = take_marks();
             k_uf_union_adds<<<grid_small, 256, 0, stream>>>(x);
             k_uf_relabel<<<grid_small, 256, 0, stream>>>(x);
             HIPCHK(hipGetLastError());
@@ -2429,6 +2482,7 @@ struct cig_engine {
     template <int W>
     void msi_relax_w() {
         MsiArgs a = msi_args(nullptr, 0, nullptr, 0);
+        a.ts = take_marks();
         advance_round(run_chain(
             [&](uint64_t tag, uint32_t seq) {
                 k_msi_consume<<<grid_msi(), kBlock, 0, stream>>>(a, a.act, prog_dev, tag, seq);
@@ -2438,7 +2492,8 @@ struct cig_engine {
         HIPCHK(hipGetLastError());
     }
 
-    void msi_relax() {
+    void msi_relax(bool last = false) {
+        last_chain = last;
         switch (weight_kind()) {
         case 0: msi_relax_w<0>(); break;
         case 1: msi_relax_w<1>(); break;
@@ -2451,8 +2506,10 @@ struct cig_engine {
     void msi_invalidate(const MsiArgs &x) {
         MsiArgs a = x;
         a.cfg = ecfg(kStageInvalidate);
+        a.ts = take_marks();
         k_msi_inval_seed<<<grid_small, kBlock, 0, stream>>>(a);
         HIPCHK(hipGetLastError());
+        a.ts = 0;
         advance_round(run_chain(
             [&](uint64_t tag, uint32_t seq) {
                 k_msi_consume<<<grid_msi(), kBlock, 0, stream>>>(a, a.pinv, prog_dev, tag, seq);
@@ -2468,8 +2525,10 @@ struct cig_engine {
         MsiArgs a = x;
         a.cfg = ecfg(kStageRepair);
         mark(8);
+        a.ts = take_marks();
         k_msi_repair<W><<<grid_small, kBlock, 0, stream>>>(a);
         mark(9);
+        a.ts = take_marks();
         scan_timed = stages_now;
         k_msi_repair_tiles<W><<<grid_small, kBlock, 0, stream>>>(a);
         k_msi_repair_done<<<grid_small, kBlock, 0, stream>>>(a);
@@ -2485,7 +2544,9 @@ struct cig_engine {
 
     template <int W>
     void msi_insert_seed(const MsiArgs &x, bool skip_affected) {
-        k_msi_insert_seed<W><<<grid_small, kBlock, 0, stream>>>(x, skip_affected ? 1u : 0u);
+        MsiArgs a = x;
+        a.ts = take_marks();
+        k_msi_insert_seed<W><<<grid_small, kBlock, 0, stream>>>(a, skip_affected ? 1u : 0u);
         HIPCHK(hipGetLastError());
     }
 
@@ -2560,13 +2621,13 @@ struct cig_engine {
         mark(3);
         if (na) msi_insert_seed<W>(x, nd != 0);
         mark(5);
-        msi_relax();
+        msi_relax(true);
         mark(4);
         end_call(st, 4);
         if (na && hctl.p->overflow_cnt) {
             recover_overflow(m);
             msi_insert_seed<W>(x, false);
-            msi_relax();
+            msi_relax(true);
             end_call(st, 4);
         }
         defer_finish(m, false);
@@ -2638,7 +2699,7 @@ struct cig_engine {
         mark(3);
         mark(5);
         pr_converge(pull);
-        mark(4);
+        mark_now(4);
         pr_residual_norm();
         mutate_finish(m);
         end_call(st, 4);
@@ -2655,11 +2716,15 @@ struct cig_engine {
         begin_call(st);
         for (int k : {1, 2, 3, 5}) mark(k);
         if (is_pr()) pr_converge();
-        else if (msk) msi_relax();
+        else if (msk) msi_relax(true);
         else if (uf_mode()) uf_all();
-        else relax();
-        mark(4);
-        if (is_pr()) pr_residual_norm();
+        else relax(true);
+        if (is_pr()) {
+            mark_now(4);
+            pr_residual_norm();
+        } else {
+            mark(4);
+        }
         end_call(st, 4);
     }
 
@@ -2777,7 +2842,8 @@ struct cig_engine {
                      cig_batch_stats *st) {
         const uint32_t k = uint32_t(dcut.size() - 1);
         if (k == 1 || nd == 0 || na == 0) return apply_device(d, nd, a, na, flags, st);
-        HIPCHK(hipEventRecord(ev[6], stream));
+        mark_always(6);
+        flush_marks();
         uint32_t bits = 10;
         while ((1ull << bits) < 2ull * na) ++bits;
         const uint64_t cap = 1ull << bits, ops = uint64_t(na) + nd;
@@ -3060,9 +3126,10 @@ struct cig_engine {
         }
         SrcList list{};
         std::memcpy(list.v, sources, size_t(k) * 4);
-        k_ms_seed<<<1, 64, 0, stream>>>(a, list, k);
-        HIPCHK(hipGetLastError());
         for (int m : {1, 2, 3, 5}) mark(m);
+        k_ms_seed<<<1, 64, 0, stream>>>(a, list, k, take_marks());
+        HIPCHK(hipGetLastError());
+        last_chain = true;
         if (bfs) ms_run<2>(a);
         else if (cfg.weight_mode == CIG_WEIGHT_HASH64) ms_run<1>(a);
         else ms_run<0>(a);
@@ -3392,8 +3459,6 @@ struct cig_engine {
         }
         if (stream) {
             (void)hipStreamSynchronize(stream);
-            for (auto &e : ev)
-                if (e) (void)hipEventDestroy(e);
             for (auto &e : rev_begin) (void)hipEventDestroy(e);
             for (auto &e : rev_end) (void)hipEventDestroy(e);
             lane.release();

@@ -45,6 +45,7 @@ struct MsiArgs {
     const uint8_t *add_skip, *del_skip;  // grouped batches: cancelled records (may be null)
     uint32_t n, k;
     uint64_t seed;
+    uint32_t ts;  // stage markers the kernel (or a chain's first round) notes
 };
 
 constexpr unsigned long long kMsiNone = ~0ull;  // value kInf, parent kNone
@@ -110,6 +111,7 @@ __device__ __forceinline__ unsigned long long msi_bits(const MsiGroup &g, bool f
 // are treated conservatively, as in the single-source path.
 __global__ __launch_bounds__(kBlock) void k_msi_inval_seed(MsiArgs a) {
     __shared__ ListStage stage;
+    stamp_marks(a.ctl, a.ts);
     const uint32_t r = a.ctl->round;
     const StagedOut<1024, 2> out{Sink{(r & 1) ? a.q1 : a.q0, &a.ctl->qcount[r % 3]}, TileSink{nullptr, &a.ctl->scount},
                                  &stage};
@@ -206,6 +208,7 @@ __global__ __launch_bounds__(kBlock) void k_msi_consume(MsiArgs a, unsigned long
         c->qcount[(r + 2) % 3] = 0;
         c->tcount[(r + 2) % 3] = 0;
         if (nq) c->rounds += 1;
+        if (seq == 1) stamp_marks(c, a.ts);
         post_progress(prog, tag, nq != 0);
     }
     const uint32_t *qin = (r & 1) ? a.q1 : a.q0;
@@ -309,6 +312,7 @@ __global__ __launch_bounds__(kBlock) void k_msi_repair(MsiArgs a) {
     __shared__ PairLds<64> lds[kWavesPerBlock];
     __shared__ uint32_t scratch[kMaxWavesPerBlock + 1];
     Ctl *c = a.ctl;
+    stamp_marks(c, a.ts);
     const uint32_t na = ld_acquire(&c->acount);
     if (na == 0) return;
     Counters ctr;
@@ -340,6 +344,7 @@ __global__ __launch_bounds__(kBlock) void k_msi_repair_tiles(MsiArgs a) {
     __shared__ PairLds<64> lds[kWavesPerBlock];
     __shared__ unsigned long long best_lds[kWavesPerBlock][kWave];
     Ctl *c = a.ctl;
+    stamp_marks(c, a.ts);
     const uint32_t nt = ld_acquire(&c->scount);
     const uint32_t lane = lane_id();
     unsigned long long *best = best_lds[wave_in_block()];
@@ -400,6 +405,7 @@ __global__ __launch_bounds__(kBlock) void k_msi_repair_done(MsiArgs a) {
 template <int W>
 __global__ __launch_bounds__(kBlock) void k_msi_insert_seed(MsiArgs a, uint32_t skip_affected) {
     __shared__ ListStage stage;
+    stamp_marks(a.ctl, a.ts);
     const uint32_t r = a.ctl->round;
     const StagedOut<1024, 2> out{Sink{(r & 1) ? a.q1 : a.q0, &a.ctl->qcount[r % 3]}, TileSink{nullptr, &a.ctl->scount},
                                  &stage};

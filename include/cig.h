@@ -147,9 +147,10 @@ typedef struct cig_config {
     uint32_t pull_blocks_per_cu; /* workgroups per CU of the PR pull kernel (at most 128) where the engine keeps the
                                     caller's ids; 0 = default (8). A renumbered engine runs one per CU */
     uint32_t kernel_timing_every; /* time one call in this many: its stage markers (the *_ms stage
-                                     fields) and, with CIG_CFG_KERNEL_TIMING, its round kernels
-                                     (each event record idles the stream a few us); total_ms is
-                                     always timed; 0 or 1 = every call */
+                                     fields), noted by the call's own kernels, and, with
+                                     CIG_CFG_KERNEL_TIMING, its round kernels (event records, each
+                                     of which idles the stream a few us); total_ms is always
+                                     timed; 0 or 1 = every call */
     uint32_t repair_delta;    /* bucket width of CIG_CFG_ORDERED_REPAIR; 0 = 128 (the reference's) */
     uint32_t pool_slack;      /* edge slots each pool gets beyond its proportional headroom (HBM
                                  without a budget: 1.25x the loaded rows' capacity; host tier:
@@ -161,8 +162,9 @@ typedef struct cig_config {
                                  expanded a round later; 0 = default (1024); <= split_degree: off */
 } cig_config;
 
-/* Per-call statistics. Times are device (HIP event) milliseconds of the
- * stage on the engine's stream; the names follow the reference's
+/* Per-call statistics. Times are milliseconds of the device's constant-rate
+ * clock, from the start of the stage's first kernel to the start of the next
+ * stage's (round_kernel_ms: HIP events); the names follow the reference's
  * [ATTR]/[DELETE-ATTR] timers (hybrid_sssp.cu:511-524, framework.cuh:2874). */
 typedef struct cig_batch_stats {
     double total_ms;          /* whole call, submit to results resident */
