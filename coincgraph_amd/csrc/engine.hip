@@ -1403,6 +1403,11 @@ struct cig_engine {
     void mutate_claims(const MutArgs &m, hipStream_t on = nullptr) {
         if (!on) on = stream;
         if (!m.nd) return;
+        if (!m.ref && (uint64_t(m.nd) << m.rev) <= kOneClaimRecords) {
+            k_del_claims<<<grid_small / 2, kBlock, 0, on>>>(m);
+            HIPCHK(hipGetLastError());
+            return;
+        }
         // tiny rows, host-tier medium rows (and in a large batch the HBM
         // medium rows with 9-16 deletes) in one launch, whose register needs
         // are alike; the HBM medium rows with up to 8 deletes keep their own
@@ -1417,16 +1422,22 @@ struct cig_engine {
 
     // claimed: mutate_claims ran already (the second stream of an overlapped
     // batch); then only the hole fixes and the adds are left.
-    void mutate_apply(const MutArgs &ma, bool claimed = false) {
+    // reset: the affected vertices' reset, where it shares the fixes' launch.
+    void mutate_apply(const MutArgs &ma, bool claimed = false, const InvalArgs *reset = nullptr) {
         MutArgs m = ma;
         if (m.nd) {
             if (!claimed) mutate_claims(m);
             m.ts = m.ref ? 0u : take_marks();  // (a captured launch takes none)
-            k_del_fix_both<<<grid_small, 256, 0, stream>>>(m, grid_small / 2);
+            if (reset)
+                k_reset_and_fix<<<grid_small + grid_small / 2, 256, 0, stream>>>(*reset, m, grid_small / 2, grid_small);
+            else
+                k_del_fix_both<<<grid_small, 256, 0, stream>>>(m, grid_small / 2);
         }
-        k_add_plan<<<grid_small, 256, 0, stream>>>(m, add_list.p, &ctl.p->add_cnt);
-        k_add_copy<<<grid_small, kBlock, 0, stream>>>(m);
-        if (m.fl.off) k_fl_release<<<grid_small, 256, 0, stream>>>(m);
+        if (m.na) {
+            k_add_plan<<<grid_small, 256, 0, stream>>>(m, add_list.p, &ctl.p->add_cnt);
+            k_add_copy<<<grid_small, kBlock, 0, stream>>>(m);
+            if (m.fl.off) k_fl_release<<<grid_small, 256, 0, stream>>>(m);
+        }
         HIPCHK(hipGetLastError());
     }
 
@@ -2053,9 +2064,7 @@ struct cig_engine {
     // the insertion seeds.
     template <int W, bool S, int QPL>
     void graph_apply_body(const MutArgs &mc, const InvalArgs &ic) {
-        k_reset_affected<<<grid_small, 256, 0, stream>>>(ic);
-        HIPCHK(hipGetLastError());
-        mutate_apply(mc, claims_beside());
+        mutate_apply(mc, claims_beside(), &ic);
         graph_repair_body<W, S, QPL>(ic, false);
     }
 
@@ -2235,10 +2244,8 @@ struct cig_engine {
             }
             // the join first: the host's wait call then overlaps the reset
             HIPCHK(hipStreamWaitEvent(stream, join_ev, 0));
-            k_reset_affected<<<grid_small, 256, 0, stream>>>(ia);
-            HIPCHK(hipGetLastError());
             mark(2);
-            mutate_apply(m, side_claims);
+            mutate_apply(m, side_claims, &ia);
             mark(1);
         } else {
             mutate_group(m);

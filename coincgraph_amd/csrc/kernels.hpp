@@ -285,6 +285,15 @@ constexpr uint32_t kDelWaveMax = 8;
 // workgroups.
 constexpr uint32_t kDelWaveMax16 = 16;
 constexpr uint64_t kMid16MinRecords = 1u << 20;
+// Batches of at most this many delete records (mirrors included; graph
+// replays, whose count the host does not know, never) claim in one launch
+// (k_del_claims): two batches of 2,000 records with a result copy 460 us in
+// three launches, 425 in one; eight of 12,500 records on 64 maintained
+// sources 8.50 and 8.35 ms. Larger ones want the waves that the kinds' own
+// register and LDS needs allow: sixteen batches of 200,000 records 10.65 ms
+// in three launches, 12.1 in one; 125,000 the same in both.
+constexpr uint64_t kOneClaimRecords = 1u << 14;
+static_assert(kOneClaimRecords < kMid16MinRecords, "k_del_claims has no 16-request rows");
 
 template <bool M16>
 __device__ __forceinline__ uint8_t del_class(uint32_t nd, uint32_t deg, bool host) {
@@ -522,8 +531,6 @@ __device__ void del_lane_body(const MutArgs &a, uint32_t bid, uint32_t nb) {
     }
 }
 
-__global__ void k_del_lane(MutArgs a) { del_lane_body(a, blockIdx.x, gridDim.x); }
-
 // Medium rows (64 < deg <= 4096 slots, at most K deletes: kDelWaveMax, or
 // kDelWaveMax16 for the HBM rows of the second kernel): one
 // 16-lane group per row (four rows per wave) reads the row once, 256 slots
@@ -701,8 +708,6 @@ __device__ void del_fix_rows_body(const MutArgs &a, uint32_t bid, uint32_t nb) {
     stat_add(&sh->missing, wave_sum64(missing));
 }
 
-__global__ void k_del_fix_rows(MutArgs a) { del_fix_rows_body(a, blockIdx.x, gridDim.x); }
-
 // Exclusive scan of a 0/1 flag over a 256-thread workgroup; *total gets the
 // sum. Contains barriers: every thread of the workgroup must call it.
 __device__ __forceinline__ uint32_t block_flag_scan(bool f, uint32_t *wsum, uint32_t &total) {
@@ -730,7 +735,7 @@ __device__ __forceinline__ uint32_t block_flag_scan(bool f, uint32_t *wsum, uint
 constexpr uint32_t kDelBloomWords = 256;
 __device__ __forceinline__ uint32_t del_bloom_bit(uint32_t x) { return (x * 0x85EBCA6Bu) >> 19; }
 
-__global__ __launch_bounds__(256) void k_del_scan(MutArgs a) {
+__device__ void del_scan_body(const MutArgs &a, uint32_t bid, uint32_t nb) {
     __shared__ uint32_t keys[kDelLdsKeys];
     // two filters, alternating by tile: a tile fills one while it clears the
     // other for the next tile, so staging needs no barrier of its own
@@ -739,7 +744,7 @@ __global__ __launch_bounds__(256) void k_del_scan(MutArgs a) {
     const uint32_t tid = threadIdx.x;
     for (uint32_t k = tid; k < kDelBloomWords; k += blockDim.x) blooms[0][k] = 0u;
     uint32_t it = 0;
-    for (uint32_t t = blockIdx.x; t < nt; t += gridDim.x, ++it) {
+    for (uint32_t t = bid; t < nt; t += nb, ++it) {
         uint32_t *bloom = blooms[it & 1u], *next = blooms[(it + 1u) & 1u];
         const DelTile dt = a.dtiles[t];
         const uint32_t bits = dt.bits, mask = (1u << bits) - 1u, to = dt.to, len = dt.len;
@@ -807,6 +812,23 @@ __global__ __launch_bounds__(256) void k_del_scan(MutArgs a) {
     }
 }
 
+__global__ __launch_bounds__(256) void k_del_scan(MutArgs a) { del_scan_body(a, blockIdx.x, gridDim.x); }
+
+// Every claim of a small batch in one launch, a quarter of the workgroups to
+// each kind of row (disjoint rows, so the kinds need no order): tiny rows,
+// host-tier medium rows, HBM medium rows, long rows. A small batch is bound
+// by the latency of each pass, not by how many waves fit: one after the other
+// the three passes of 1000 deletes took 47 us, together 21.
+__global__ __launch_bounds__(kBlock) void k_del_claims(MutArgs a) {
+    const uint32_t nb = gridDim.x / 4u, part = blockIdx.x / nb, bid = blockIdx.x - part * nb;
+    switch (part) {
+    case 0: del_lane_body(a, bid, nb); break;
+    case 1: del_rows_body<2, true>(a, bid, nb); break;
+    case 2: del_rows_body<4, false>(a, bid, nb); break;
+    default: del_scan_body(a, bid, gridDim.x - 3u * nb); break;
+    }
+}
+
 // Compaction of rows with more than kDelThreadFix deletes (or a table), one
 // workgroup per row: with k holes the row shrinks to deg-k and the live
 // slots of the last k positions move into the holes below deg-k (O(k)
@@ -870,8 +892,6 @@ __device__ void del_fix_body(const MutArgs &a, uint32_t bid, uint32_t nb) {
         stat_add(&sh->missing, missing);
     }
 }
-
-__global__ __launch_bounds__(256) void k_del_fix(MutArgs a) { del_fix_body(a, blockIdx.x, gridDim.x); }
 
 // Both hole fixes in one launch (they own disjoint rows): the first `split`
 // workgroups take the rows fixed by one thread each, the others one row per
@@ -1296,12 +1316,12 @@ __global__ __launch_bounds__(kBlock) void k_inval_round(InvalArgs a, uint64_t *p
 
 // reset_affected_values (driver.cuh:418-433): affected vertices restart from
 // the initial value (CC: own label), and all of them form the next frontier.
-__global__ void k_reset_affected(InvalArgs a) {
+__device__ void reset_affected_body(const InvalArgs &a, uint32_t bid, uint32_t nb) {
     __shared__ uint32_t scratch[kMaxWavesPerBlock + 1];
     const uint32_t cnt = ld_acquire(&a.ctl->acount);
     const uint32_t r = a.ctl->round;
     uint32_t *q = (r & 1) ? a.q1 : a.q0;
-    for (uint32_t base = blockIdx.x * blockDim.x; base < cnt; base += gthreads()) {
+    for (uint32_t base = bid * blockDim.x; base < cnt; base += nb * blockDim.x) {
         const uint32_t i = base + threadIdx.x;
         bool push = false;
         uint32_t v = 0;
@@ -1312,6 +1332,19 @@ __global__ void k_reset_affected(InvalArgs a) {
         }
         block_append(push, v, q, &a.ctl->qcount[r % 3], scratch);
     }
+}
+
+__global__ void k_reset_affected(InvalArgs a) { reset_affected_body(a, blockIdx.x, gridDim.x); }
+
+// The reset beside the hole fixes of the same batch: the one writes vertex
+// state and the frontier, the other rows, so where no wave runs between them
+// they share a launch (first `split` workgroups: the reset; then, as in
+// k_del_fix_both, up to `split2` the rows fixed by one thread each).
+__global__ __launch_bounds__(256) void k_reset_and_fix(InvalArgs a, MutArgs m, uint32_t split, uint32_t split2) {
+    stamp_marks(a.ctl, m.ts);
+    if (blockIdx.x < split) reset_affected_body(a, blockIdx.x, split);
+    else if (blockIdx.x < split2) del_fix_rows_body(m, blockIdx.x - split, split2 - split);
+    else del_fix_body(m, blockIdx.x - split2, gridDim.x - split2);
 }
 
 // SeedAddedEdgeFrontier (framework.cuh:238-294): each inserted (u,v) offers
