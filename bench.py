@@ -254,7 +254,7 @@ def main(argv=None):
                     help="PageRank: rounds with at least n/this many frontier vertices gather "
                          "(cig_config.pr_pull_divisor; 0 = default)")
     ap.add_argument("--pull-blocks", type=int, default=0,
-                    help="PageRank: workgroups per CU of the pull kernels (0 = default)")
+                    help="PageRank: workgroups per CU of the pull kernel of an engine that keeps the caller ids (0 = default)")
     ap.add_argument("--edges-per-lane", type=int, default=0,
                     help="edges each lane keeps in flight: 4, 8 or 16 (0 = default)")
     ap.add_argument("--pr-push", action="store_true",
@@ -400,8 +400,8 @@ def main(argv=None):
     # when no round gathered). Its duration comes from the HIP event pair the
     # engine records around every launch on its own stream; its algorithmic
     # bytes are its pass's (stage_bytes) spread over all its launches (no-op
-    # lookahead rounds, and for k_pr_pull the sparse rounds it leaves to the
-    # scatter, included, as rocprofv3 counts them).
+    # lookahead rounds, and for k_pr_pull the sparse rounds, which it scatters,
+    # included, as rocprofv3 counts them).
     # Only the batches whose round kernels were timed enter (one in TIMING_EVERY;
     # every batch for PageRank).
     timed = [s for s in stats if s["round_launches"]]

@@ -1165,9 +1165,9 @@ struct cig_engine {
                 },
                 cfg.pr_max_rounds, "PageRank"));
         } else {
-            // a dense round gathers along the incoming rows (k_pr_pull +
-            // k_pr_pull_long), a sparse one scatters; each kernel checks
-            // the round's frontier size and returns when it is not its form
+            // a dense round gathers along the incoming rows, a sparse one
+            // scatters: k_pr_pull reads the round's frontier size and takes
+            // the round's form
             if (!plan_ready) pull_plan(a, nullptr);
             k_pr_degrees<<<grid_small, 256, 0, stream>>>(rows.p, n, odeg.p);
             advance_round(run_chain(

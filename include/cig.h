@@ -407,8 +407,8 @@ cig_status cig_query(cig_engine *e, uint32_t algo, const uint32_t *sources, uint
 /* No counterpart in the reference. For callers that cannot allocate (code
  * under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc): cig_query without any allocation. The run's working memory
- * (vertex-major distances, source masks, stamps: 4*round_up(nsrc,4) + 28
- * bytes per vertex, 36 for BFS) lives in a fixed device array of
+ * (vertex-major distances, source masks and their snapshots: room for
+ * 4*round_up(nsrc,4) + 28 bytes per vertex, 36 for BFS, is asked for) lives in a fixed device array of
  * CIG_NOALLOC_SCRATCH_BYTES that each GPU holds from library load to process
  * exit; sources are passed by value; the distances are written to the
  * caller's device memory dist_device (nsrc*n words, source-major, as
