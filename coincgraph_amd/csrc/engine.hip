@@ -244,7 +244,11 @@ constexpr uint32_t kQplDefault = 2;  // quads (4 slots) per lane and step
 constexpr uint32_t kPullDivisorDefault = 4096;
 // The mask pays where the contributions' lines come from HBM: at 2^22
 // vertices (16 MB of contributions) a masked sweep takes 350 us, 270 without.
-constexpr uint32_t kPullMaskDivisor = 4;
+// At 2^25 a sweep without it takes 3.4 ms whatever the frontier, one with it
+// 4.35 at n/4 and less from about n/40 on: a batch of 500,000 + 500,000 takes
+// 156.5 ms at a divisor of 4, 149.7 at 12, 147.5 at 20, 147.0 at 40, 148.0 at
+// 80 and 149.5 at 160.
+constexpr uint32_t kPullMaskDivisor = 40;
 constexpr uint32_t kPullMaskMin = 1u << 24;
 constexpr uint32_t kPullBlocksPerCu = 8;
 // BFS queries: rounds whose frontier holds at least n / kMsPullDivisor
