@@ -242,14 +242,15 @@ constexpr uint32_t kQplDefault = 2;  // quads (4 slots) per lane and step
 // all incoming rows costs less than scattering with atomics from a frontier
 // of n/4096 hub-heavy vertices.)
 constexpr uint32_t kPullDivisorDefault = 4096;
-// The mask pays where the contributions' lines come from HBM: at 2^22
-// vertices (16 MB of contributions) a masked sweep takes 350 us, 270 without.
-// At 2^25 a sweep without it takes 3.4 ms whatever the frontier, one with it
-// 4.35 at n/4 and less from about n/40 on: a batch of 500,000 + 500,000 takes
-// 156.5 ms at a divisor of 4, 149.7 at 12, 147.5 at 20, 147.0 at 40, 148.0 at
-// 80 and 149.5 at 160.
-constexpr uint32_t kPullMaskDivisor = 40;
-constexpr uint32_t kPullMaskMin = 1u << 24;
+// A sweep without the mask test takes the same time whatever the frontier;
+// one with it reads a bit per slot first and pays once few gathers are left.
+// At 2^25 vertices 3.4 ms without, 4.35 with at n/4, less from about n/40 on:
+// a batch of 500,000 + 500,000 takes 156.5 ms at a divisor of 4, 147.5 at 20,
+// 147.0 at 40, 148.0 at 80, 149.5 at 160. At 2^22 two batches of 62,500 +
+// 62,500 take 32.9 ms without the test, 31.3 at 40, 31.1 at 160, 31.4 to 32.0
+// at 640; a solve of 1,000,003 vertices takes the same either way.
+constexpr uint32_t kPullMaskDivisor = 64;
+constexpr uint32_t kPullMaskMin = 1u << 20;
 constexpr uint32_t kPullBlocksPerCu = 8;
 // BFS queries: rounds whose frontier holds at least n / kMsPullDivisor
 // vertices gather along the incoming rows, in graphs whose rows are all in HBM

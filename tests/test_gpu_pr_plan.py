@@ -72,3 +72,28 @@ def test_pull_plan_edges(n, flags, divisor, cap):
             settle(e.apply_batch(dels, adds))
             oracle_apply(og, dels, adds)
             _check(e, og, f"batch {b}")
+
+
+@pytest.mark.parametrize("flags", [0, cg.CFG_PR_KEEP_IDS])
+@pytest.mark.parametrize("n", [1 << 20, (1 << 20) + 1])
+def test_mask_rule_edge(n, flags):
+    """The vertex count from which sparse sweeps test the source mask: a solve
+    whose frontier shrinks through every form, then a batch whose rounds start
+    sparse."""
+    print(f"[gpu-case] mask rule n={n} flags={flags}", flush=True)
+    g = _graph(n, n)
+    og = oracle_graph(g)
+    rng = np.random.default_rng(n)
+    with cg.Engine("pr", pr_epsilon=1e-7, pr_max_rounds=1000, flags=flags) as e:
+        e.load_graph(g)
+        e.init_graph()
+        assert e.start()["converged"]
+        _check(e, og, "initial")
+        off, dst = og.csr()
+        at = rng.permutation(int(off[-1]))[:3000]
+        u = (np.searchsorted(off, at, side="right") - 1).astype(np.uint32)
+        dels = cg.edges_array(u, dst[at])
+        adds = cg.edges_array(rng.integers(0, n, 3000).astype(np.uint32), rng.integers(0, n, 3000).astype(np.uint32))
+        assert e.apply_batch(dels, adds)["converged"]
+        oracle_apply(og, dels, adds)
+        _check(e, og, "batch")
