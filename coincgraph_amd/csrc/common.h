@@ -65,6 +65,7 @@ struct Ctl {
     alignas(kCtlLine) uint32_t flist[3];   // list entries written by the scan of such a frontier
     uint32_t round;        // next absolute round to run
     uint32_t converged;
+    uint32_t parked;       // round whose frontier a query has set aside (k_clear_frontier)
     alignas(kCtlLine) uint32_t done;  // workgroups finished in the current round kernel
     uint32_t iround;       // invalidation: first round of the running chain
     uint32_t istart[3];    // invalidation: where round slot k's frontier starts in the affected list

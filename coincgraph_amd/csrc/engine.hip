@@ -830,6 +830,7 @@ struct cig_engine {
         sync();
         loaded = true;
         initialized = false;
+        frontier_pending = frontier_parked = false;
     }
 
     // Tile lists hold at most one round's worth of tiles: every row of the
@@ -1095,6 +1096,30 @@ struct cig_engine {
         }
     }
 
+    // Whether the queues may hold a frontier that no call has run: after
+    // init, after a call that a round cap stopped and after one that failed.
+    bool frontier_pending = false, frontier_was_pending = false, frontier_parked = false;
+
+    // Sets the pending frontier aside for a query (see k_clear_frontier).
+    void park_frontier() {
+        if (!is_pr() && !msk && !uf_mode()) k_park_tiles<<<grid_small, 256, 0, stream>>>(ctl.p, stamp.p, t0.p, t1.p);
+        k_clear_frontier<<<1, 64, 0, stream>>>(ctl.p, 1u);
+        HIPCHK(hipGetLastError());
+        frontier_parked = true;
+    }
+
+    // Lists it again, for the next call of the engine's own. (A union-find
+    // engine runs no frontier.)
+    void unpark_frontier() {
+        frontier_parked = false;
+        frontier_pending = true;
+        k_clear_frontier<<<1, 64, 0, stream>>>(ctl.p, 0u);
+        if (!uf_mode())
+            k_list_frontier<<<grid_small, 256, 0, stream>>>(ctl.p, is_pr() ? kMarkQueued : msk ? kMarkAct : kMarkStamp,
+                                                            stamp.p, msi_act.p, q0.p, q1.p, n);
+        HIPCHK(hipGetLastError());
+    }
+
     PrArgs pr_args(uint32_t max_rounds) {
         PrArgs a{};
         a.ctl = ctl.p;
@@ -1195,6 +1220,8 @@ struct cig_engine {
         if (!loaded) throw HipError(CIG_ESTATE, "cig_load_csr must come first");
         flush_finish();  // the last batch's clear needs its counters, which the reset zeroes
         reset_ctl(false);
+        frontier_pending = true;
+        frontier_parked = false;
         if (is_pr()) {
             k_init_pr<<<grid_small, 256, 0, stream>>>(rank.p, comp.p, res.p, stamp.p, q1.p, n, ctl.p);
         } else if (cfg.algo == CIG_ALGO_CC) {
@@ -1233,6 +1260,9 @@ struct cig_engine {
             rounds_pending = 0;
             advance_round(by);
         }
+        if (frontier_parked) unpark_frontier();  // a query that ended by an exception
+        frontier_was_pending = frontier_pending;
+        frontier_pending = true;  // until end_call has seen that it is not
         if (!quick) flush_finish();
         scan_timed = false;
         overlapped = false;
@@ -1294,6 +1324,7 @@ struct cig_engine {
 
     void end_call(cig_batch_stats *st, int marks) {
         end_and_read_ctl();
+        frontier_pending = relax_pending(*hctl.p);
         if (hctl.p->pr_invalid) throw HipError(CIG_EINTERNAL, "PR non-finite rank/residual");
         if (!is_pr() && !cfg.max_rounds) {
             const uint32_t r = hctl.p->round;
@@ -3117,6 +3148,7 @@ struct cig_engine {
     // has begun the call and cleared mem (query_clear).
     void query_run(uint32_t algo, const uint32_t *sources, uint32_t k, const QueryMem &mem) {
         const bool bfs = algo == CIG_ALGO_BFS;
+        if (frontier_was_pending) park_frontier();
         MsArgs a{};
         a.ctl = ctl.p;
         a.rows = rows.p;
@@ -3148,6 +3180,11 @@ struct cig_engine {
         mark(4);
     }
 
+    void query_end(cig_batch_stats *st) {
+        end_call(st, 4);
+        if (frontier_parked) unpark_frontier();
+    }
+
     // The results go straight to each caller's buffer (no merged host copy).
     void query(uint32_t algo, const uint32_t *sources, uint32_t k, const QueryOut *outs, size_t nouts,
                cig_batch_stats *st) {
@@ -3177,7 +3214,7 @@ struct cig_engine {
         const QueryMem m{ms_dist.p, ms_mark.p, ms_snap.p};
         query_clear(algo, k, m);
         query_run(algo, sources, k, m);
-        end_call(st, 4);
+        query_end(st);
     }
 
     // Source-major results of the last query_compute of k sources into the
@@ -3233,7 +3270,7 @@ struct cig_engine {
         query_run(algo, sources, k, m);
         k_ms_gather<0><<<grid_small, kBlock, 0, stream>>>(m.dist, n, stride, k, dist_dev);
         HIPCHK(hipGetLastError());
-        end_call(st, 4);
+        query_end(st);
     }
 
     void copy_out(void *out, const void *dev, uint64_t bytes) { lane.copy(out, dev, bytes); }

@@ -1708,6 +1708,43 @@ __global__ void k_advance_round(Ctl *c, uint32_t by) {
     if (threadIdx.x == 0 && blockIdx.x == 0) c->round += by;
 }
 
+// A query runs its rounds through the engine's queues, so a frontier pending
+// there (of an engine that is initialised and not solved yet, or stopped by a
+// round cap) is set aside first and listed again afterwards. It needs no copy:
+// the frontier is the vertices whose mark is set, and a query touches no mark.
+enum : uint32_t { kMarkStamp = 0, kMarkQueued = 1, kMarkAct = 2 };  // stamp = the round; PR's flag; msi.hpp's act
+
+// The owners of pending tiles join the frontier: their whole rows are expanded
+// again, which changes no fixed point, and the tiles need not be kept.
+__global__ void k_park_tiles(Ctl *c, uint32_t *stamp, const Tile *t0, const Tile *t1) {
+    const uint32_t r = c->round, nt = c->tcount[r % 3];
+    const Tile *tiles = (r & 1) ? t1 : t0;
+    for (uint32_t i = gthread(); i < nt; i += gthreads()) stamp[tiles[i].v] = r;
+}
+
+// No frontier in any slot; park != 0 notes the round of the one set aside.
+__global__ void k_clear_frontier(Ctl *c, uint32_t park) {
+    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    if (park) c->parked = c->round;
+    for (int i = 0; i < 3; ++i) c->qcount[i] = c->tcount[i] = c->fscan[i] = c->flist[i] = 0;
+}
+
+// Lists the frontier set aside as the current round's.
+__global__ void k_list_frontier(Ctl *c, uint32_t kind, uint32_t *stamp, const unsigned long long *act, uint32_t *q0,
+                                uint32_t *q1, uint32_t n) {
+    __shared__ uint32_t scratch[kMaxWavesPerBlock + 1];
+    const uint32_t r = c->round, from = c->parked;
+    for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += gthreads()) {
+        const uint32_t v = base + threadIdx.x;
+        bool on = v < n;
+        if (kind == kMarkAct) on = on && act[v] != 0ull;
+        else if (kind == kMarkQueued) on = on && stamp[v] != 0u;
+        else on = on && stamp[v] == from;
+        if (on && kind == kMarkStamp) stamp[v] = r;
+        block_append(on, v, (r & 1) ? q1 : q0, &c->qcount[r % 3], scratch);
+    }
+}
+
 // ---------------------------------------------------------- PageRank rounds
 // Pull plan of one solve. Incoming rows of up to kPullSplit slots are listed
 // by size class: class c holds the rows of up to 4 << c slots, which 1 << c
@@ -2667,7 +2704,7 @@ __global__ __launch_bounds__(kBlock) void k_ms_consume(MsArgs a, uint64_t *prog,
                     on = (a.all & ~x.x) != 0ull;  // this vertex gathers
                     if (on) row = a.in_rows[v];
                 } else {
-                    on = m != 0ull;
+                    on = !scan || m != 0ull;  // every listed vertex leaves a snapshot
                 }
             } else {
                 m = a.act[v];
