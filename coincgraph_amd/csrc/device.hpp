@@ -742,13 +742,17 @@ __device__ void expand_tiles(const Op &op, const ExpandCfg &cfg, const Tile *til
 // six workgroups' LDS on a CU: 16-source SSSP over 2^20 vertices 9.2 ms, 9.5
 // with 512.
 constexpr uint32_t kPairSlots = 128;
+// Rows of more slots are always cut in these passes, whatever split_degree and
+// tile_len say: 64 rows of fewer slots than this and 64 sources hold fewer than
+// 2^32 items, and a row or tile (at most twice as long) at most 2^26.
+constexpr uint32_t kPairSplitMax = 1u << 19;
 template <int NG>
 struct PairLds {
     uint32_t pref[kWave];   // exclusive scan of the rows' item counts
     uint32_t spref[kWave];  // and of their slot counts
     uint32_t v[kWave];
     uint32_t cnt[kWave];    // groups of the row's mask
-    uint32_t magic[kWave];  // ceil(2^32 / cnt): item / cnt is exact below 2^26 items a row
+    uint32_t magic[kWave];  // ceil(2^32 / cnt): item / cnt is exact for the items of a row, below 2^26
     uint32_t offlo[kWave], offhi[kWave];
     unsigned long long mask[kWave];
     uint8_t perm[NG > 1 ? kWave : 1][NG];  // the mask's groups in order
@@ -922,7 +926,7 @@ __host__ __device__ __forceinline__ uint32_t pair_tile_len(const ExpandCfg &c) {
 // workgroup-uniform call, one reservation per workgroup.
 __device__ __forceinline__ void pair_cut(const ExpandCfg &cfg, uint32_t tl, uint32_t v, const Row &row, bool on,
                                          Tile *tiles, uint32_t *count, uint32_t *scratch) {
-    const uint32_t nt = on && row.deg >= cfg.split ? (row.deg + tl - 1) / tl : 0u;
+    const uint32_t nt = on && row.deg >= cfg.split ? (row.deg - 1) / tl + 1 : 0u;
     const uint32_t at = block_reserve<uint32_t>(nt, count, scratch);
     for (uint32_t j = 0; j < nt; ++j) {
         Tile t;

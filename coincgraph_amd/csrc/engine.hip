@@ -393,6 +393,13 @@ struct cig_engine {
         return uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(grid_small, g)));
     }
     ExpandCfg ecfg(uint32_t stage) const { return ExpandCfg{pools(), split, tile_len, stage, stats.p}; }
+    // of the passes over (edge, source) pairs
+    ExpandCfg ecfg_pairs(uint32_t stage) const {
+        ExpandCfg c = ecfg(stage);
+        c.split = std::min(split, kPairSplitMax);
+        c.tile_len = std::min(tile_len, 2 * kPairSplitMax);
+        return c;
+    }
     uint32_t weight_kind() const {
         switch (cfg.algo) {
         case CIG_ALGO_BFS: return 2;
@@ -834,10 +841,11 @@ struct cig_engine {
     }
 
     // Tile lists hold at most one round's worth of tiles: every row of the
-    // round at most once, so sum(deg)/tile_len + rows >= split.
+    // round at most once, so sum(deg)/tile_len + rows >= split (of a pass over
+    // pairs: at most slots / its split).
     void ensure_tiles() {
         const uint64_t slots = hbm_slots + host_slots;
-        const uint64_t need = slots / tile_len + slots / split + 1024;
+        const uint64_t need = slots / tile_len + slots / std::min(split, kPairSplitMax) + 1024;
         if (need <= tile_cap) return;
         t0.alloc(need);
         t1.alloc(need);
@@ -2472,7 +2480,7 @@ struct cig_engine {
         x.q1 = q1.p;
         x.tiles = t0.p;
         x.alist = alist.p;
-        x.cfg = ecfg(kStagePropagate);
+        x.cfg = ecfg_pairs(kStagePropagate);
         x.dels = d;
         x.nd = nd;
         x.adds = a;
@@ -2548,7 +2556,7 @@ struct cig_engine {
     // every affected vertex.
     void msi_invalidate(const MsiArgs &x) {
         MsiArgs a = x;
-        a.cfg = ecfg(kStageInvalidate);
+        a.cfg = ecfg_pairs(kStageInvalidate);
         a.ts = take_marks();
         k_msi_inval_seed<<<grid_small, kBlock, 0, stream>>>(a);
         HIPCHK(hipGetLastError());
@@ -2566,7 +2574,7 @@ struct cig_engine {
     template <int W>
     void msi_repair(const MsiArgs &x) {
         MsiArgs a = x;
-        a.cfg = ecfg(kStageRepair);
+        a.cfg = ecfg_pairs(kStageRepair);
         mark(8);
         a.ts = take_marks();
         k_msi_repair<W><<<grid_small, kBlock, 0, stream>>>(a);
@@ -3158,7 +3166,7 @@ struct cig_engine {
         a.q0 = q0.p;
         a.q1 = q1.p;
         a.tiles = t0.p;
-        a.cfg = ecfg(kStagePropagate);
+        a.cfg = ecfg_pairs(kStagePropagate);
         a.n = n;
         a.stride = (k + 3u) & ~3u;
         a.seed = cfg.weight_seed;

@@ -134,7 +134,8 @@ typedef struct cig_config {
     uint32_t segments;        /* accepted for flag compatibility (1..512) */
     uint32_t block_size;      /* threads per workgroup; 0 = tuned default */
     uint32_t edges_per_lane;  /* edges each lane keeps in flight: 4, 8 or 16 (whole 16-B quads); 0 = tuned default */
-    uint32_t split_degree;    /* rows at least this long are split into tiles; 0 = default */
+    uint32_t split_degree;    /* rows at least this long are split into tiles; 0 = default. Passes over
+                                 several sources split rows of 2^19 slots and more in any case */
     uint32_t max_rounds;      /* traversal round cap per launch; 0 = unlimited (exact) */
     uint32_t pr_max_rounds;   /* rounds per solve; the reference's flag allows
                                  1..100 (hybrid_pr.cu:22), the library 1..10^6 */
