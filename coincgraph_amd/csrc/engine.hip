@@ -167,16 +167,26 @@ struct CopyLane {
             own_stream = true;
         }
     }
+    // The ring's buffers and events; false when there is no memory for them.
+    bool have_ring() {
+        try {
+            for (unsigned b = 0; b < kRing; ++b) {
+                if (!bounce[b].p) bounce[b].alloc(kChunk);
+                if (!ev[b]) HIPCHK(hipEventCreateWithFlags(&ev[b], hipEventDisableTiming));
+            }
+            return true;
+        } catch (const HipError &x) {
+            if (x.code != CIG_ENOMEM) throw;
+            (void)hipGetLastError();
+            return false;
+        }
+    }
     // Copies `bytes` from device memory to `out`; returns with the copy complete.
     void copy(void *out, const void *dev, uint64_t bytes) {
-        if (bytes <= kDirect) {
+        if (bytes <= kDirect || !have_ring()) {
             HIPCHK(hipMemcpyAsync(out, dev, bytes, hipMemcpyDeviceToHost, stream));
             HIPCHK(hipStreamSynchronize(stream));
             return;
-        }
-        for (unsigned b = 0; b < kRing; ++b) {
-            if (!bounce[b].p) bounce[b].alloc(kChunk);
-            if (!ev[b]) HIPCHK(hipEventCreateWithFlags(&ev[b], hipEventDisableTiming));
         }
         const uint64_t chunks = (bytes + kChunk - 1) / kChunk;
         std::atomic<uint64_t> ready{0};    // chunks in their buffers; ~0: give up
@@ -3396,13 +3406,15 @@ struct cig_engine {
             }
             return;
         }
+        // 4 B a vertex on their way out: mutation scratch (nrows >= n words),
+        // free between calls, so that reading results takes no device memory
+        uint32_t *const out_words = overflow.p;
         // a renumbered engine's words go back to the caller's order on the device
         auto words = [&](const uint32_t *src) {
             if (renum) {
-                grow(out_words, n);
-                k_permute_words<<<grid_small, 256, 0, stream>>>(src, perm_d.p, n, out_words.p);
+                k_permute_words<<<grid_small, 256, 0, stream>>>(src, perm_d.p, n, out_words);
                 HIPCHK(hipGetLastError());
-                src = out_words.p;
+                src = out_words;
             }
             copy_out(out, src, uint64_t(n) * 4);
         };
@@ -3429,12 +3441,10 @@ struct cig_engine {
             copy_out(out, ms_out.p, words * 4);
             return;
         }
-        grow(out_words, n);
-        k_state_words<<<grid_small, 256, 0, stream>>>(state.p, n, field == CIG_FIELD_VALUE ? 1u : 0u, out_words.p);
+        k_state_words<<<grid_small, 256, 0, stream>>>(state.p, n, field == CIG_FIELD_VALUE ? 1u : 0u, out_words);
         HIPCHK(hipGetLastError());
-        copy_out(out, out_words.p, uint64_t(n) * 4);
+        copy_out(out, out_words, uint64_t(n) * 4);
     }
-    DBuf<uint32_t> out_words;  // a result field on its way out (4 B a vertex)
 
     // Rows [first, first+n) as CSR: the outgoing rows (first = 0) or the
     // incoming index (first = n).

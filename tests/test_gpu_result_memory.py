@@ -1,0 +1,57 @@
+"""Reading results takes no device memory: values, parents and a renumbered
+PageRank engine's fields, of 4 MiB and more, leave the free device memory as
+it was."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import coincgraph_amd as cg
+from tests.test_zz_no_alloc import _hip
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _need_gpu():
+    if cg.device_count() < 1:
+        pytest.skip("no HIP device")
+
+
+def _free(hip):
+    free, total = C.c_size_t(), C.c_size_t()
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def _chain(n):
+    """0 -> 1 -> 2 and no other edge."""
+    off = np.full(n + 1, 2, dtype=np.uint64)
+    off[0], off[1] = 0, 1
+    return cg.HostGraph(n, off, np.array([1, 2], dtype=np.uint32))
+
+
+@pytest.mark.parametrize("algo", ["bfs", "pr"])
+def test_results_take_no_device_memory(algo):
+    print(f"[gpu-case] result memory {algo}", flush=True)
+    hip = _hip()
+    read = (lambda e: (e.values(), e.parents())) if algo == "bfs" else (lambda e: (e.values(), e.residuals()))
+    with cg.Engine(algo) as warm:  # the kernels and the copy path have run once
+        warm.load_graph(_chain(1 << 20))
+        warm.init_graph(0)
+        warm.start()
+        read(warm)
+    n = 1 << 23
+    with cg.Engine(algo) as e:
+        e.load_graph(_chain(n))
+        e.init_graph(0)
+        e.start()
+        before = _free(hip)
+        a, b = read(e)
+        assert _free(hip) == before
+    if algo == "bfs":
+        assert a[:4].tolist() == [0, 1, 2, cg.INF] and (a[3:] == cg.INF).all()
+        assert b[:4].tolist() == [cg.INF, 0, 1, cg.INF] and (b[3:] == cg.INF).all()
+    else:
+        assert np.allclose(a[:4], [0.15, 0.2775, 0.385875, 0.15], rtol=1e-6, atol=0) and (a[3:] == a[0]).all()
+        assert (np.abs(b) <= 1e-6).all()
