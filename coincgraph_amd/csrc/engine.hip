@@ -333,7 +333,6 @@ struct cig_engine {
     DBuf<unsigned long long> amask;  // active-source mask of the pull passes
     DBuf<uint32_t> odeg;             // out-degrees for the dense consume of one solve
     DBuf<unsigned long long> adm_hist, adm_acc;  // cache admission: capacity per score, sums
-    uint64_t ptile_cap = 0;
     DBuf<uint64_t> cnt64, gofs;
     DBuf<uint32_t> rslot;  // per record of a call: rank within its row's deletes / adds
     DBuf<uint32_t> touched, grouped, small_list, mid_list, mid16_list, big_list, add_list, overflow;
@@ -1178,16 +1177,16 @@ struct cig_engine {
         const uint64_t slots = hbm_slots + host_slots;
         const uint64_t rows_long = std::min<uint64_t>(n, slots / kPullSplit);
         const uint64_t need = slots / kPullTile + rows_long + 1;
-        // sized by n: a later cig_load_csr may bring a larger graph
+        const uint64_t rows_multi = std::min<uint64_t>(n, slots / kPullTile) + 1;
+        // each by its own count: a later cig_load_csr may bring a graph that
+        // needs more of one and less of another, and an allocation may fail
         if (amask.count < (uint64_t(n) + 63) / 64) amask.alloc((uint64_t(n) + 63) / 64);
         if (odeg.count < n) odeg.alloc(n);
         if (pent.count < n) pent.alloc(n);
         if (!pcnt.p) pcnt.alloc(kPlanBlocks * kPlanLists);
-        if (need <= ptile_cap) return;
-        ptiles.alloc(need);
-        tpart.alloc(need);
-        prow.alloc(std::min<uint64_t>(n, slots / kPullTile) + 1);
-        ptile_cap = need;
+        if (ptiles.count < need) ptiles.alloc(need);
+        if (tpart.count < need) tpart.alloc(need);
+        if (prow.count < rows_multi) prow.alloc(rows_multi);
     }
 
     // Runtime::Converge (pr_residual.cuh:171-187): at most pr_max_rounds
@@ -2383,10 +2382,8 @@ struct cig_engine {
     bool uf_mode() const { return (cfg.flags & CIG_CFG_CC_UNION_REPAIR) && cfg.algo == CIG_ALGO_CC; }
 
     UfArgs uf_args(const cig_edge *d, uint32_t nd, const cig_edge *a, uint32_t na) {
-        if (uf.count < n) {
-            uf.alloc(n);
-            uroot.alloc(n);
-        }
+        if (uf.count < n) uf.alloc(n);
+        if (uroot.count < n) uroot.alloc(n);
         UfArgs x{};
         x.ctl = ctl.p;
         x.rows = rows.p;
@@ -3223,10 +3220,8 @@ struct cig_engine {
         query_check(algo, sources, k);
         const uint32_t stride = (k + 3u) & ~3u;
         if (ms_dist.count < uint64_t(n) * stride) ms_dist.alloc(uint64_t(n) * stride);
-        if (ms_mark.count < 2ull * n) {
-            ms_mark.alloc(2ull * n);
-            ms_snap.alloc(n);
-        }
+        if (ms_mark.count < 2ull * n) ms_mark.alloc(2ull * n);
+        if (ms_snap.count < n) ms_snap.alloc(n);
         if (ms_out.count < uint64_t(n) * k) ms_out.alloc(uint64_t(n) * k);
         begin_call(st);
         const QueryMem m{ms_dist.p, ms_mark.p, ms_snap.p};

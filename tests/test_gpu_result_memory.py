@@ -55,3 +55,26 @@ def test_results_take_no_device_memory(algo):
     else:
         assert np.allclose(a[:4], [0.15, 0.2775, 0.385875, 0.15], rtol=1e-6, atol=0) and (a[3:] == a[0]).all()
         assert (np.abs(b) <= 1e-6).all()
+
+
+def test_pagerank_of_a_second_graph_with_more_long_rows():
+    """An engine's second graph needs fewer tiles than its first but has more
+    incoming rows of several tiles."""
+    print("[gpu-case] PageRank of a second graph", flush=True)
+    from tests.helpers import oracle_graph, pr_errors
+    rng = np.random.default_rng(95)
+
+    def graph(n, u, v):
+        order = np.argsort(u, kind="stable")
+        off = np.zeros(n + 1, dtype=np.uint64)
+        off[1:] = np.cumsum(np.bincount(u, minlength=n))
+        return cg.HostGraph(n, off, v[order].astype(np.uint32))
+
+    with cg.Engine("pr", pr_epsilon=1e-7, pr_max_rounds=1000, pool_slack=1) as e:
+        for n, rows, length in ((3, 3, 700_000), (2000, 60, 3000)):
+            v = np.concatenate([np.repeat(np.arange(rows), length), rng.integers(0, n, n)])
+            g = graph(n, rng.integers(0, n, len(v)), v)
+            e.load_graph(g)
+            e.init_graph()
+            assert e.start()["converged"]
+            assert pr_errors(e.values(), oracle_graph(g).pagerank()[0])[0] <= 1e-6, n
