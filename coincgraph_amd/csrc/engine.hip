@@ -322,7 +322,7 @@ struct cig_engine {
     DBuf<PullRow> prow;
     DBuf<PullEntry> pent;
     DBuf<uint32_t> pcnt;
-    DBuf<float> tpart;
+    DBuf<unsigned long long> tpart;
     DBuf<unsigned long long> fl_off;  // host-tier free blocks by class (FreeList), when the tier holds rows
     DBuf<int> fl_cnt;
     static constexpr uint32_t kFlCap = 1u << 20;  // blocks listed per class
@@ -1185,7 +1185,10 @@ struct cig_engine {
         if (pent.count < n) pent.alloc(n);
         if (!pcnt.p) pcnt.alloc(kPlanBlocks * kPlanLists);
         if (ptiles.count < need) ptiles.alloc(need);
-        if (tpart.count < need) tpart.alloc(need);
+        if (tpart.count < need) {
+            tpart.alloc(need);
+            fill32(reinterpret_cast<uint32_t *>(tpart.p), 2 * need, 0u);
+        }
         if (prow.count < rows_multi) prow.alloc(rows_multi);
     }
 
