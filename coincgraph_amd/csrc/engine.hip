@@ -753,6 +753,7 @@ struct cig_engine {
         hbm_pool.alloc(hbm_slots);
         host_pool.alloc(host_slots);
         host_pool_dev = host_pool.device_ptr();
+        if (short_results() && mapped_words.count < n) mapped_words.alloc(n, hipHostMallocCoherent | hipHostMallocMapped);
         if (host_need) {
             if (!fl_off.p) {
                 fl_off.alloc(uint64_t(kFlClasses) * kFlCap);
@@ -3291,6 +3292,21 @@ struct cig_engine {
 
     void copy_out(void *out, const void *dev, uint64_t bytes) { lane.copy(out, dev, bytes); }
 
+    // Where a kernel forms the words of a result field of n vertices: in mapped
+    // host memory up to the direct copy's size (a field of 1,000 vertices is
+    // read in 13 us, with a copy of the runtime in 24; 32,768: 18 and 30;
+    // 524,288: 117 and 140), else in mutation scratch (nrows >= n words, free
+    // between calls) for the lane's ring, so that reading results takes no
+    // device memory.
+    HBuf<uint32_t> mapped_words;
+    bool short_results() const { return uint64_t(n) * 4 <= CopyLane::kDirect; }
+    uint32_t *word_space() const { return short_results() ? mapped_words.device_ptr() : overflow.p; }
+    void copy_words(void *out, const uint32_t *words) {
+        if (!short_results()) return copy_out(out, words, uint64_t(n) * 4);
+        sync();
+        std::memcpy(out, mapped_words.p, size_t(n) * 4);
+    }
+
     // ------------------------------------------------------------ cache
     // Sort-based admission (compute_hot_vertices + confirm_candidate_batch,
     // framework.cuh:605-729): rows by score descending (stable: ties by id),
@@ -3404,17 +3420,13 @@ struct cig_engine {
             }
             return;
         }
-        // 4 B a vertex on their way out: mutation scratch (nrows >= n words),
-        // free between calls, so that reading results takes no device memory
-        uint32_t *const out_words = overflow.p;
         // a renumbered engine's words go back to the caller's order on the device
         auto words = [&](const uint32_t *src) {
-            if (renum) {
-                k_permute_words<<<grid_small, 256, 0, stream>>>(src, perm_d.p, n, out_words);
-                HIPCHK(hipGetLastError());
-                src = out_words;
-            }
-            copy_out(out, src, uint64_t(n) * 4);
+            if (!renum) return copy_out(out, src, uint64_t(n) * 4);
+            uint32_t *to = word_space();
+            k_permute_words<<<grid_for(n, 1), 256, 0, stream>>>(src, perm_d.p, n, to);
+            HIPCHK(hipGetLastError());
+            copy_words(out, to);
         };
         if (field == CIG_FIELD_HOTNESS) {
             words(score.p);
@@ -3439,9 +3451,10 @@ struct cig_engine {
             copy_out(out, ms_out.p, words * 4);
             return;
         }
-        k_state_words<<<grid_small, 256, 0, stream>>>(state.p, n, field == CIG_FIELD_VALUE ? 1u : 0u, out_words);
+        uint32_t *to = word_space();
+        k_state_words<<<grid_for(n, 1), 256, 0, stream>>>(state.p, n, field == CIG_FIELD_VALUE ? 1u : 0u, to);
         HIPCHK(hipGetLastError());
-        copy_out(out, out_words, uint64_t(n) * 4);
+        copy_words(out, to);
     }
 
     // Rows [first, first+n) as CSR: the outgoing rows (first = 0) or the
@@ -3502,7 +3515,7 @@ struct cig_engine {
         gi->hbm_pool_used = hctl.p->pool_tail[0];
         gi->host_pool_slots = host_slots;
         gi->host_pool_used = hctl.p->pool_tail[1];
-        gi->host_pinned_bytes = host_slots * 4 + sizeof(Ctl);
+        gi->host_pinned_bytes = host_slots * 4 + sizeof(Ctl) + mapped_words.count * 4;
         gi->device_bytes = hbm_slots * 4 + rows.bytes() + state.bytes() + rank.bytes() * 4 + q0.bytes() * 2 +
                            stamp.bytes() + aff.bytes() + alist.bytes() + hot.bytes() * 3 + t0.bytes() * 2 +
                            cnt64.bytes() * 3 + touched.bytes() * 5 + pieces.bytes() + grouped.bytes() +

@@ -78,3 +78,28 @@ def test_pagerank_of_a_second_graph_with_more_long_rows():
             e.init_graph()
             assert e.start()["converged"]
             assert pr_errors(e.values(), oracle_graph(g).pagerank()[0])[0] <= 1e-6, n
+
+
+@pytest.mark.parametrize("n", [1, 2, 255, 257, 40000, 524287, 524288, 524289])
+def test_results_around_the_mapped_size(n):
+    """Short results are formed in host memory, longer ones copied."""
+    print(f"[gpu-case] short results n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    off = np.zeros(n + 1, dtype=np.uint64)
+    off[1:] = np.cumsum(rng.integers(0, 4, n))
+    g = cg.HostGraph(n, off, rng.integers(0, n, int(off[-1])).astype(np.uint32))
+    from tests.helpers import check_traversal, oracle_graph, pr_errors
+    og = oracle_graph(g)
+    with cg.Engine("sssp") as e:
+        e.load_graph(g)
+        e.init_graph(0)
+        e.start()
+        for _ in range(2):
+            check_traversal(e, og, "sssp", 0)
+    for flags in (0, cg.CFG_PR_KEEP_IDS):
+        with cg.Engine("pr", pr_epsilon=1e-7, pr_max_rounds=1000, flags=flags) as e:
+            e.load_graph(g)
+            e.init_graph()
+            assert e.start()["converged"]
+            assert pr_errors(e.values(), og.pagerank()[0])[0] <= 1e-6
+            assert (np.abs(e.residuals()) <= 1e-7).all()
