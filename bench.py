@@ -256,7 +256,7 @@ def main(argv=None):
     ap.add_argument("--pull-blocks", type=int, default=0,
                     help="PageRank: workgroups per CU of the pull kernel of an engine that keeps the caller ids (0 = default)")
     ap.add_argument("--edges-per-lane", type=int, default=0,
-                    help="edges each lane keeps in flight: 4, 8 or 16 (0 = default)")
+                    help="edges each lane keeps in flight in single-source propagation and repair: 4, 8 or 16 (0 = default)")
     ap.add_argument("--pr-push", action="store_true",
                     help="PageRank: scatter every round with atomics (keeps no incoming rows)")
     ap.add_argument("--serve-seconds", type=float, default=30.0, help="serving: arrival window (s)")

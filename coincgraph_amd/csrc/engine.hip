@@ -132,7 +132,7 @@ struct HBuf {  // pinned host memory (hipHostMalloc; never hipHostRegister)
 // of host threads moves each finished one out (and takes the page faults of a
 // buffer the caller has not touched yet). The runtime's own copy to pageable
 // memory runs at about 10 GB/s here; 16 MB take 0.5 ms this way instead of
-// 1.5, 67 MB 1.6 instead of 6.3. Results below kDirect keep the plain copy,
+// 1.5, 67 MB 1.6 instead of 6.3. Results up to kDirect keep the plain copy,
 // which is done before a team would have started. The engine's lane uses the
 // engine stream; the serving loop has a second lane, so that a query's
 // results leave the device while the next update group runs.
@@ -248,7 +248,8 @@ constexpr uint32_t kAdaptSplitDefault = 1024;
 constexpr uint32_t kQplDefault = 2;  // quads (4 slots) per lane and step
 // PR rounds whose frontier holds at least n / kPullDivisorDefault vertices
 // run in pull form; below n / kPullMaskDivisor the pull tests the
-// active-source mask before each gather. (R-MAT scale 25: a masked sweep of
+// active-source mask before each gather, in graphs of more than kPullMaskMin
+// vertices. (R-MAT scale 25: a masked sweep of
 // all incoming rows costs less than scattering with atomics from a frontier
 // of n/4096 hub-heavy vertices.)
 constexpr uint32_t kPullDivisorDefault = 4096;
@@ -256,9 +257,12 @@ constexpr uint32_t kPullDivisorDefault = 4096;
 // one with it reads a bit per slot first and pays once few gathers are left.
 // At 2^25 vertices 3.4 ms without, 4.35 with at n/4, less from about n/40 on:
 // a batch of 500,000 + 500,000 takes 156.5 ms at a divisor of 4, 147.5 at 20,
-// 147.0 at 40, 148.0 at 80, 149.5 at 160. At 2^22 two batches of 62,500 +
-// 62,500 take 32.9 ms without the test, 31.3 at 40, 31.1 at 160, 31.4 to 32.0
-// at 640; a solve of 1,000,003 vertices takes the same either way.
+// 147.0 at 40, 147.2 at 64, 148.0 at 80, 149.5 at 160. At 2^22 two batches of
+// 62,500 + 62,500 take 32.9 ms without the test, 31.3 at 40, 31.2 at 64, 31.1
+// at 160, 31.4 to 32.0 at 640. Up to 2^20 vertices the contributions fit the
+// 4 MB of an XCD's L2, where a gather costs no more than the test before it:
+// without and with it a solve of 2^18 vertices takes 3.71 and 3.90 ms, a batch
+// of 1000 + 1000 on 2^12 2.19 and 2.34, a solve of 2^20 8.13 and 8.12.
 constexpr uint32_t kPullMaskDivisor = 64;
 constexpr uint32_t kPullMaskMin = 1u << 20;
 constexpr uint32_t kPullBlocksPerCu = 8;
@@ -267,7 +271,13 @@ constexpr uint32_t kPullBlocksPerCu = 8;
 // (a gather reads the rows of every vertex that misses a source, which the
 // host link would pay for). 64 sources of 200,003 vertices, all rounds: n / 4
 // 307 us, n / 16 233, n / 64 252 (a round of n / 40 vertices gathers in 29 us
-// and pushes in 9), never 465.
+// and pushes in 9), never 465. Never, n / 4, n / 16 and n / 64 in us, R-MAT
+// with 16 edges a vertex: 2^12 vertices, 1 source 96, 105, 93, 89; 2^16, 1
+// source 146, 149, 137, 135, 64 sources 318, 300, 226, 226; 2^20, 1 source
+// 481, 459, 458, 317, 16 sources 1203, 828, 803, 569; 2^22, 8 sources 3628,
+// 2182, 2180, 1688. Uniform random, 2^20: 1 source 611, 342, 340, 473, 16
+// sources 1692, 750, 752, 887. A grid of 2^16, 64 sources: 16,668, 16,729,
+// 10,120, 9513. 2^17 vertices with 4 edges each, 1 source: 165, 175, 176, 175.
 constexpr uint32_t kMsPullDivisor = 16;
 
 }  // namespace
@@ -3251,9 +3261,10 @@ struct cig_engine {
     }
 
     // Byte offsets of a run's working memory inside the no-allocation scratch
-    // array, each 256-B aligned: distances, marks (two words a vertex),
-    // snapshots. The documented size (36 bytes a vertex beside the distances
-    // for BFS, 28 for SSSP) is what a run may need, and is kept as the limit.
+    // array, each 256-B aligned: distances, marks (two words a vertex for BFS,
+    // one for SSSP), snapshots. A run uses 24 (BFS) or 16 (SSSP) bytes a vertex
+    // beside the distances; the documented limit asks for 4 more, so that the
+    // sizes that are refused stay the same.
     static uint64_t noalloc_layout(uint32_t nv, uint32_t k, bool bfs, uint64_t off[3]) {
         auto up = [](uint64_t x) { return (x + 255) & ~uint64_t(255); };
         const uint64_t stride = (k + 3u) & ~3u, word = up(uint64_t(nv) * 8);
@@ -3521,7 +3532,8 @@ struct cig_engine {
                            cnt64.bytes() * 3 + touched.bytes() * 5 + pieces.bytes() + grouped.bytes() +
                            rec_dels.bytes() * 2 + s_adds.bytes() + s_dels.bytes() + filt.bytes() +
                            htoff.bytes() + hcnt.bytes() + hkeys.bytes() + hcnts.bytes() + dtiles.bytes() +
-                           stats.bytes();
+                           stats.bytes() + pent.bytes() + pcnt.bytes() + ptiles.bytes() + prow.bytes() +
+                           tpart.bytes() + odeg.bytes() + amask.bytes();
     }
 
     ~cig_engine() {

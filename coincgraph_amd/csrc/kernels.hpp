@@ -531,8 +531,9 @@ __device__ void del_lane_body(const MutArgs &a, uint32_t bid, uint32_t nb) {
     }
 }
 
-// Medium rows (64 < deg <= 4096 slots, at most K deletes: kDelWaveMax, or
-// kDelWaveMax16 for the HBM rows of the second kernel): one
+// Medium rows (HBM: 64 < deg <= 4096 slots, host tier: up to 4096, none
+// included; at most K deletes: kDelWaveMax, or kDelWaveMax16 for the HBM rows
+// of the second kernel): one
 // 16-lane group per row (four rows per wave) reads the row once, 256 slots
 // a step, against all of the row's requested destinations, which the
 // group's lanes hold in registers (a destination requested twice is two

@@ -133,7 +133,9 @@ typedef struct cig_config {
                                  instead) */
     uint32_t segments;        /* accepted for flag compatibility (1..512) */
     uint32_t block_size;      /* threads per workgroup; 0 = tuned default */
-    uint32_t edges_per_lane;  /* edges each lane keeps in flight: 4, 8 or 16 (whole 16-B quads); 0 = tuned default */
+    uint32_t edges_per_lane;  /* edges each lane keeps in flight: 4, 8 or 16 (whole 16-B quads); 0 = tuned default.
+                                 Single-source propagation and repair, and the union-find hooking; queries,
+                                 several sources and PageRank take theirs by the kernel */
     uint32_t split_degree;    /* rows at least this long are split into tiles; 0 = default. Passes over
                                  several sources split rows of 2^19 slots and more in any case */
     uint32_t max_rounds;      /* traversal round cap per launch; 0 = unlimited (exact) */
@@ -409,7 +411,7 @@ cig_status cig_query(cig_engine *e, uint32_t algo, const uint32_t *sources, uint
  * under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc): cig_query without any allocation. The run's working memory
  * (vertex-major distances, source masks and their snapshots: room for
- * 4*round_up(nsrc,4) + 28 bytes per vertex, 36 for BFS, is asked for) lives in a fixed device array of
+ * 4*round_up(nsrc,4) + 20 bytes per vertex, 28 for BFS, is asked for) lives in a fixed device array of
  * CIG_NOALLOC_SCRATCH_BYTES that each GPU holds from library load to process
  * exit; sources are passed by value; the distances are written to the
  * caller's device memory dist_device (nsrc*n words, source-major, as
