@@ -459,6 +459,8 @@ struct cig_engine {
         pub.alloc(1, hipHostMallocCoherent | hipHostMallocMapped);
         std::memset(pub.p, 0, sizeof(CtlPub));
         pub_dev = pub.device_ptr();
+        mapped_words.alloc(kMappedWords, hipHostMallocCoherent | hipHostMallocMapped);
+        mapped_dev = mapped_words.device_ptr();
         stats.alloc(kStatShards);
         HIPCHK(hipMemsetAsync(stats.p, 0, stats.bytes(), stream));
         std::memset(hctl.p, 0, sizeof(Ctl));
@@ -763,7 +765,6 @@ struct cig_engine {
         hbm_pool.alloc(hbm_slots);
         host_pool.alloc(host_slots);
         host_pool_dev = host_pool.device_ptr();
-        if (short_results() && mapped_words.count < n) mapped_words.alloc(n, hipHostMallocCoherent | hipHostMallocMapped);
         if (host_need) {
             if (!fl_off.p) {
                 fl_off.alloc(uint64_t(kFlClasses) * kFlCap);
@@ -3303,19 +3304,39 @@ struct cig_engine {
 
     void copy_out(void *out, const void *dev, uint64_t bytes) { lane.copy(out, dev, bytes); }
 
-    // Where a kernel forms the words of a result field of n vertices: in mapped
-    // host memory up to the direct copy's size (a field of 1,000 vertices is
-    // read in 13 us, with a copy of the runtime in 24; 32,768: 18 and 30;
-    // 524,288: 117 and 140), else in mutation scratch (nrows >= n words, free
-    // between calls) for the lane's ring, so that reading results takes no
-    // device memory.
+    // A result field of n vertices to host memory, without taking device memory:
+    // the words at src (null: `form(first, count, to)` enqueues the kernel that
+    // forms them). Three ways by length; us for a field that a kernel forms, an
+    // engine's first and a later one:
+    //   vertices                              1,000  98,304  262,144  300,000  524,288
+    //   mapped host memory, a buffer a time   27/15  162/44  242/95            374/195
+    //   scratch, hipMemcpy                                   200/170  125/105  185/165
+    //   scratch, copy on the engine stream    40/26  210/192 470/453  590/520  208/165
+    // (1,000,000 on the engine stream through the lane's ring: 820/215; by
+    // hipMemcpy 300/290 for words that need no kernel, 2,000,000 540 and 290.)
+    static constexpr uint32_t kMappedWords = 1u << 16, kFormMapped = 1u << 18;
     HBuf<uint32_t> mapped_words;
-    bool short_results() const { return uint64_t(n) * 4 <= CopyLane::kDirect; }
-    uint32_t *word_space() const { return short_results() ? mapped_words.device_ptr() : overflow.p; }
-    void copy_words(void *out, const uint32_t *words) {
-        if (!short_results()) return copy_out(out, words, uint64_t(n) * 4);
+    uint32_t *mapped_dev = nullptr;
+    template <class Form>
+    void copy_words(void *out, const uint32_t *src, Form form) {
+        if (n <= kFormMapped) {
+            for (uint32_t at = 0; at < n; at += kMappedWords) {
+                const uint32_t cnt = std::min(kMappedWords, n - at);
+                form(at, cnt, mapped_dev);
+                HIPCHK(hipGetLastError());
+                sync();
+                std::memcpy(static_cast<uint32_t *>(out) + at, mapped_words.p, size_t(cnt) * 4);
+            }
+            return;
+        }
+        if (!src) {
+            src = overflow.p;  // mutation scratch (nrows >= n words), free between calls
+            form(0u, n, overflow.p);
+            HIPCHK(hipGetLastError());
+        }
+        if (uint64_t(n) * 4 > CopyLane::kDirect) return copy_out(out, src, uint64_t(n) * 4);
         sync();
-        std::memcpy(out, mapped_words.p, size_t(n) * 4);
+        HIPCHK(hipMemcpy(out, src, size_t(n) * 4, hipMemcpyDeviceToHost));
     }
 
     // ------------------------------------------------------------ cache
@@ -3433,11 +3454,10 @@ struct cig_engine {
         }
         // a renumbered engine's words go back to the caller's order on the device
         auto words = [&](const uint32_t *src) {
-            if (!renum) return copy_out(out, src, uint64_t(n) * 4);
-            uint32_t *to = word_space();
-            k_permute_words<<<grid_for(n, 1), 256, 0, stream>>>(src, perm_d.p, n, to);
-            HIPCHK(hipGetLastError());
-            copy_words(out, to);
+            copy_words(out, renum ? nullptr : src, [&](uint32_t at, uint32_t cnt, uint32_t *to) {
+                k_permute_words<<<grid_for(cnt, 1), 256, 0, stream>>>(renum ? src : src + at,
+                                                                     renum ? perm_d.p + at : nullptr, cnt, to);
+            });
         };
         if (field == CIG_FIELD_HOTNESS) {
             words(score.p);
@@ -3462,10 +3482,9 @@ struct cig_engine {
             copy_out(out, ms_out.p, words * 4);
             return;
         }
-        uint32_t *to = word_space();
-        k_state_words<<<grid_for(n, 1), 256, 0, stream>>>(state.p, n, field == CIG_FIELD_VALUE ? 1u : 0u, to);
-        HIPCHK(hipGetLastError());
-        copy_words(out, to);
+        copy_words(out, nullptr, [&](uint32_t at, uint32_t cnt, uint32_t *to) {
+            k_state_words<<<grid_for(cnt, 1), 256, 0, stream>>>(state.p + at, cnt, field == CIG_FIELD_VALUE ? 1u : 0u, to);
+        });
     }
 
     // Rows [first, first+n) as CSR: the outgoing rows (first = 0) or the

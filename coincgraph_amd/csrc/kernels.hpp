@@ -2929,9 +2929,10 @@ __global__ void k_state_words(const uint64_t *state, uint32_t n, uint32_t high, 
     for (uint32_t v = gthread(); v < n; v += gthreads()) out[v] = uint32_t(high ? state[v] >> 32 : state[v]);
 }
 
-// out[v] = src[perm[v]]: a renumbered engine's words in the caller's order.
+// out[v] = src[perm[v]]: a renumbered engine's words in the caller's order
+// (perm null: as they are).
 __global__ void k_permute_words(const uint32_t *src, const uint32_t *perm, uint32_t n, uint32_t *out) {
-    for (uint32_t v = gthread(); v < n; v += gthreads()) out[v] = src[perm[v]];
+    for (uint32_t v = gthread(); v < n; v += gthreads()) out[v] = src[perm ? perm[v] : v];
 }
 
 // Plain streaming copy (16 B per lane per step): the HBM reference point for
