@@ -1472,7 +1472,7 @@ struct cig_engine {
         if (!on) on = stream;
         if (!m.nd) return;
         if (!m.ref && (uint64_t(m.nd) << m.rev) <= kOneClaimRecords) {
-            k_del_claims<<<grid_small / 2, kBlock, 0, on>>>(m);
+            k_del_claims<<<std::max(4u, grid_small / 2 & ~3u), kBlock, 0, on>>>(m);
             HIPCHK(hipGetLastError());
             return;
         }

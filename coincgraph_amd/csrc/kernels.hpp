@@ -819,10 +819,11 @@ __global__ __launch_bounds__(256) void k_del_scan(MutArgs a) { del_scan_body(a, 
 // each kind of row (disjoint rows, so the kinds need no order): tiny rows,
 // host-tier medium rows, HBM medium rows, long rows. A small batch is bound
 // by the latency of each pass, not by how many waves fit: one after the other
-// the three passes of 1000 deletes took 47 us, together 21. At least four
-// workgroups; the long rows' share takes the remainder.
+// the three passes of 1000 deletes took 47 us, together 21. The
+// grid is a multiple of four workgroups (a remainder would take scan tiles
+// twice; testing for it here costs the fourth wave a SIMD: 131 registers).
 __global__ __launch_bounds__(kBlock) void k_del_claims(MutArgs a) {
-    const uint32_t nb = gridDim.x / 4u, part = min(blockIdx.x / nb, 3u), bid = blockIdx.x - part * nb;
+    const uint32_t nb = gridDim.x / 4u, part = blockIdx.x / nb, bid = blockIdx.x - part * nb;
     switch (part) {
     case 0: del_lane_body(a, bid, nb); break;
     case 1: del_rows_body<2, true>(a, bid, nb); break;
