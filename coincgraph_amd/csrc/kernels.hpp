@@ -2428,9 +2428,10 @@ __device__ __forceinline__ void frontier_count(Ctl *c, uint32_t slot, uint32_t j
 // per CU that wrote the frontier's list, searched every slot's row and added
 // quads up in LDS; now 56 / 265. Two sets of rows in flight per wave: one 62 /
 // 280, four 76 / 335 (their lines displace each other in L1). Without HUB: 81
-// / 360.
+// / 360; it is held to the 128 registers of four waves a SIMD (132 and three
+// waves: a solve of 2^20 vertices 12.6 -> 13.2 ms).
 template <bool HUB>
-__global__ __launch_bounds__(HUB ? kPullHubBlock : kBlock) void k_pr_pull(PrArgs a, uint32_t seq) {
+__global__ __launch_bounds__(HUB ? kPullHubBlock : kBlock, 4) void k_pr_pull(PrArgs a, uint32_t seq) {
     constexpr uint32_t B = HUB ? kPullHubBlock : kBlock;
     struct ScatterLds {
         WaveLds w[B / kWave];
