@@ -459,8 +459,6 @@ struct cig_engine {
         pub.alloc(1, hipHostMallocCoherent | hipHostMallocMapped);
         std::memset(pub.p, 0, sizeof(CtlPub));
         pub_dev = pub.device_ptr();
-        mapped_words.alloc(kMappedWords, hipHostMallocCoherent | hipHostMallocMapped);
-        mapped_dev = mapped_words.device_ptr();
         stats.alloc(kStatShards);
         HIPCHK(hipMemsetAsync(stats.p, 0, stats.bytes(), stream));
         std::memset(hctl.p, 0, sizeof(Ctl));
@@ -765,6 +763,11 @@ struct cig_engine {
         hbm_pool.alloc(hbm_slots);
         host_pool.alloc(host_slots);
         host_pool_dev = host_pool.device_ptr();
+        if (!mapped_words.p) mapped_words.alloc(2 * kMappedWords, hipHostMallocCoherent | hipHostMallocMapped);
+        mapped_dev = mapped_words.device_ptr();
+        // its pages are touched here, where they cost nothing beside the load,
+        // instead of by the first result (1.4 us a page)
+        std::memset(mapped_words.p, 0, size_t(std::min(n, 2 * kMappedWords)) * 4);
         if (host_need) {
             if (!fl_off.p) {
                 fl_off.alloc(uint64_t(kFlClasses) * kFlCap);
@@ -3305,38 +3308,40 @@ struct cig_engine {
     void copy_out(void *out, const void *dev, uint64_t bytes) { lane.copy(out, dev, bytes); }
 
     // A result field of n vertices to host memory, without taking device memory:
-    // the words at src (null: `form(first, count, to)` enqueues the kernel that
-    // forms them). Three ways by length; us for a field that a kernel forms, an
-    // engine's first and a later one:
-    //   vertices                              1,000  98,304  262,144  300,000  524,288
-    //   mapped host memory, a buffer a time   27/15  162/44  242/95            374/195
-    //   scratch, hipMemcpy                                   200/170  125/105  185/165
-    //   scratch, copy on the engine stream    40/26  210/192 470/453  590/520  208/165
-    // (1,000,000 on the engine stream through the lane's ring: 820/215; by
-    // hipMemcpy 300/290 for words that need no kernel, 2,000,000 540 and 290.)
-    static constexpr uint32_t kMappedWords = 1u << 16, kFormMapped = 1u << 18;
-    HBuf<uint32_t> mapped_words;
+    // the words at src (null: a kernel has to form them), which
+    // `form(first, count, to)` enqueues a kernel for. Up to the direct copy's size
+    // they are formed in mapped host memory, in two buffers by turns: the copies
+    // of the runtime take that long for some sizes and several times as long for
+    // others. us for a field that a kernel forms, an engine's first and a later one:
+    //   vertices                           1,000  98,304   262,144  400,000  524,288
+    //   mapped host memory                 27/15  59/40    109/83   144/128  197/157
+    //   scratch, copy on the engine stream 40/26  210/192  470/450  740/480  208/165
+    //   scratch, hipMemcpy                                 200/170  150/115  185/165
+    // (500,000 by hipMemcpy: 110 in one program, 830 in another.) Longer fields
+    // are formed in scratch for the lane's ring (1,000,000: 820/215).
+    static constexpr uint32_t kMappedWords = 1u << 16;
+    HBuf<uint32_t> mapped_words;  // two buffers
     uint32_t *mapped_dev = nullptr;
     template <class Form>
     void copy_words(void *out, const uint32_t *src, Form form) {
-        if (n <= kFormMapped) {
-            for (uint32_t at = 0; at < n; at += kMappedWords) {
-                const uint32_t cnt = std::min(kMappedWords, n - at);
-                form(at, cnt, mapped_dev);
+        if (uint64_t(n) * 4 > CopyLane::kDirect) {
+            if (!src) {
+                src = overflow.p;  // mutation scratch (nrows >= n words), free between calls
+                form(0u, n, overflow.p);
                 HIPCHK(hipGetLastError());
-                sync();
-                std::memcpy(static_cast<uint32_t *>(out) + at, mapped_words.p, size_t(cnt) * 4);
             }
-            return;
+            return copy_out(out, src, uint64_t(n) * 4);
         }
-        if (!src) {
-            src = overflow.p;  // mutation scratch (nrows >= n words), free between calls
-            form(0u, n, overflow.p);
+        auto part = [&](uint32_t at) { return std::min(kMappedWords, n - at); };
+        uint32_t half = 0;
+        form(0u, part(0), mapped_dev);
+        for (uint32_t at = 0; at < n; at += kMappedWords, half ^= kMappedWords) {
             HIPCHK(hipGetLastError());
+            sync();
+            if (n - at > kMappedWords)  // formed while this part is copied
+                form(at + kMappedWords, part(at + kMappedWords), mapped_dev + (half ^ kMappedWords));
+            std::memcpy(static_cast<uint32_t *>(out) + at, mapped_words.p + half, size_t(part(at)) * 4);
         }
-        if (uint64_t(n) * 4 > CopyLane::kDirect) return copy_out(out, src, uint64_t(n) * 4);
-        sync();
-        HIPCHK(hipMemcpy(out, src, size_t(n) * 4, hipMemcpyDeviceToHost));
     }
 
     // ------------------------------------------------------------ cache
